@@ -328,6 +328,23 @@ int selection_chunk(const double* scores, int n, int points, int resolution, int
                     int* missing, uint8_t* chosen, uint8_t* nodes, int* tree, const int* offsets,
                     const int* sizes, int levels, int chunk, int64_t* stats, int* trace, uint64_t stream);
 
+/* A head start for selection_chunk when the order of the choices is not wanted: the state the rule
+ * reaches after most of its choices, found in parallel.  No counterpart in the reference.
+ * odie_selection_relax queues `launches` relaxation passes (first != 0: from the start) on the node
+ * levels in workspace (device, odie_selection_bulk_workspace(points) bytes); pass i sets flags[i]
+ * (device int64, cleared by the caller) to 1 when it raised a level.  Once a pass has left its flag
+ * at 0, odie_selection_bulk puts the state of selection_init (missing, chosen, nodes, tree, stats)
+ * to the one selection_chunk reaches with at most cap - 4 nodes used (chosen cells' missing 0), or
+ * leaves it as it is when the scores give no such point (a negative or non-finite score, scores
+ * above 2^1000, ties reaching across it); selection_chunk then goes on from either, to the same
+ * chosen cells, nodes and iteration count.  points = align8(n), n = resolution^2, 8 <= cap <= points. */
+int64_t odie_selection_bulk_workspace(int points);
+int odie_selection_relax(const double* scores, int n, int points, int resolution, int normalized, void* workspace,
+                         int64_t workspace_bytes, int first, int64_t* flags, int launches, uint64_t stream);
+int odie_selection_bulk(const double* scores, int n, int points, int resolution, int cap, int normalized,
+                        int* missing, uint8_t* chosen, uint8_t* nodes, int* tree, int64_t* stats, void* workspace,
+                        int64_t workspace_bytes, uint64_t stream);
+
 /* ---------------------------------------------------------------------------------------
  * Fused Adam over n parameters: master fp32 (updated), half_copy fp16 (nullable; receives
  * fp16(master) in the same pass), grad fp32 or fp16 carrying loss_scale, moments m, v fp32.

@@ -54,6 +54,9 @@ SIGNATURES = {
     'odie_selection_tree_ints': ([_I], _I64),
     'selection_init': ([_P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _U64], _I),
     'selection_chunk': ([_P, _I, _I, _I, _I, C.c_bool, _P, _P, _P, _P, _P, _P, _I, _I, _P, _P, _U64], _I),
+    'odie_selection_bulk_workspace': ([_I], _I64),
+    'odie_selection_relax': ([_P, _I, _I, _I, _I, _P, _I64, _I, _P, _I, _U64], _I),
+    'odie_selection_bulk': ([_P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I64, _U64], _I),
     'odie_mlp_forward': ([_P, _I64, _I, _P, _P, _U64], _I),
     'odie_mlp_train': ([_P, _I64, _I, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _U64], _I),
     'odie_mlp_train_planes': ([_P, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _U64], _I),

@@ -68,3 +68,54 @@ def test_large_grid_with_device_resident_tree_levels():
 def test_zero_scores_still_fill_capacity():
     values = np.zeros(32 * 32)
     _check(values, 32, 256)
+
+
+def _bulk_scores(kind, resolution):
+    cells = resolution * resolution
+    values = synth.uniform(13, 'bulk' + kind, cells).astype(np.float64)
+    if kind == 'ties':
+        return _scores(13, cells, True)
+    if kind == 'thirds':      # score/3, score/2 and score/4 of different cells meet up to rounding
+        return np.array([1.0, 2.0, 3.0, 4.0, 6.0, 1 / 3, 2 / 3])[(values * 7).astype(int)]
+    if kind == 'patches':     # flat zero ground with a few bright blocks, as a mostly settled residual
+        plane = values.reshape(resolution, resolution) * 1e-3
+        plane[: resolution // 2] = 0.0
+        plane[resolution // 4: resolution // 3, resolution // 4:] += 5.0
+        return plane.reshape(-1)
+    if kind == 'chain':       # one long row of cells each freed by the last: levels cross every tile
+        plane = np.full((resolution, resolution), 1e-9)
+        plane[resolution // 2] = 1.0 + 1e-6 * np.arange(resolution)
+        plane[resolution // 2, 0] = 4.5
+        return plane.reshape(-1)
+    if kind == 'nan':
+        values[cells // 3] = np.nan
+    if kind == 'negative':
+        values[::7] *= -1.0
+    if kind == 'huge':
+        values[::5] *= 1e304
+    if kind == 'tiny':
+        values *= 5e-324 * 64
+    return values
+
+
+@pytest.mark.parametrize('resolution', [8, 31, 32, 33, 64, 65, 129, 200])
+@pytest.mark.parametrize('kind', ['uniform', 'ties', 'thirds', 'patches', 'chain', 'nan', 'negative', 'huge', 'tiny'])
+def test_bulk_start_equals_one_choice_at_a_time(kind, resolution):
+    """Without a trace most choices are found in parallel; with one each is made in its turn."""
+    scores = torch.from_numpy(_bulk_scores(kind, resolution)).cuda()
+    points = align8(resolution * resolution)
+    for cap in sorted({64, points // 64 * 8, points // 16 * 8, points - 8, points}):
+        for normalize in (True, False):
+            selected, nodes, iterations, _ = select_device(scores, resolution, cap, normalize, trace=True)
+            got = select_device(scores, resolution, cap, normalize)
+            what = (kind, resolution, cap, normalize)
+            assert got[2] == iterations, what
+            assert torch.equal(got[0], selected) and torch.equal(got[1], nodes), what
+
+
+def test_bulk_start_against_the_oracle():
+    values = _scores(17, 150 * 150, False)
+    selected, nodes, iterations = oracle.select_benefit_cost(values, 150, 4000)
+    got = select_device(torch.from_numpy(values).cuda(), 150, 4000)
+    assert got[2] == iterations
+    assert np.array_equal(got[0].cpu().numpy(), selected) and np.array_equal(got[1].cpu().numpy(), nodes)
