@@ -89,15 +89,17 @@ __device__ inline void grid_corners(const DevLevel& lv, float x, float y, uint32
 // from +0, on both features at once (v_pk_fma_f16); entries and the result are fp16 pairs
 // (feature 0 in the low half).  The forward's arithmetic (odie/packed_kernels.cu:52-62).
 __device__ inline uint32_t half2_level(const uint32_t g[4], const float w[4]) {
-    __half2 acc = __half2(__float2half(0.0f), __float2half(0.0f));
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const __half2 value = __halves2half2(bits_to_half(static_cast<uint16_t>(g[k] & 0xffffu)),
-                                             bits_to_half(static_cast<uint16_t>(g[k] >> 16)));
-        acc = __hfma2(__float2half2_rn(keep_fp32(w[k])), value, acc);
-    }
-    return static_cast<uint32_t>(half_to_bits(__low2half(acc))) |
-           (static_cast<uint32_t>(half_to_bits(__high2half(acc))) << 16);
+    typedef _Float16 pair __attribute__((ext_vector_type(2)));
+    typedef float float_pair __attribute__((ext_vector_type(2)));
+    // the weights converted two at a time (v_cvt_pk_f16_f32)
+    const pair w01 = __builtin_convertvector((float_pair){keep_fp32(w[0]), keep_fp32(w[1])}, pair);
+    const pair w23 = __builtin_convertvector((float_pair){keep_fp32(w[2]), keep_fp32(w[3])}, pair);
+    pair acc = {};
+    acc = __builtin_elementwise_fma((pair){w01.x, w01.x}, __builtin_bit_cast(pair, g[0]), acc);
+    acc = __builtin_elementwise_fma((pair){w01.y, w01.y}, __builtin_bit_cast(pair, g[1]), acc);
+    acc = __builtin_elementwise_fma((pair){w23.x, w23.x}, __builtin_bit_cast(pair, g[2]), acc);
+    acc = __builtin_elementwise_fma((pair){w23.y, w23.y}, __builtin_bit_cast(pair, g[3]), acc);
+    return __builtin_bit_cast(uint32_t, acc);
 }
 
 template <bool HALF>

@@ -5,7 +5,7 @@ predictions bit for bit, over ragged ranges and with tiles that have no expert. 
 scoring pipeline (score_image): per-cell totals bit-exact against the oracle's residual of the
 fused predictions, the top tiles against the oracle's ranking, the mse against torch's expression;
 both the streamed form (odie_reconstruct + score_chunk) and the fused one (odie_reconstruct_scores,
-a wave per cell)."""
+one or several waves per cell)."""
 import numpy as np
 import pytest
 import torch
@@ -14,6 +14,7 @@ import oracle
 from odie_amd import synth
 from odie_amd.decoder import Decoder
 from odie_amd.experts import ExpertGrid, route
+from odie_amd.gpu_residual import DeviceScores
 from odie_amd.reconstruction import reconstruct, score_image
 from odie_amd.selection import topk_tiles
 
@@ -116,3 +117,66 @@ def test_device_image_on_the_gpu_equals_numpy():
     expected = synth.image(7, 300, 170)
     got = synth.image_device(7, 300, 170, device='cuda', rows=64).cpu().numpy()
     assert np.array_equal(got, expected)
+
+
+@pytest.mark.parametrize('shape,resolution,tile', [
+    ((330, 330), None, 33),      # 1089 pixels: several waves per cell, ragged rounds; 100 cells
+    ((640, 640), None, 32),      # 1024 pixels exactly; more cells than CUs
+    ((96, 1100), 3, None),       # tall and narrow native cells across tile bounds
+    ((40, 40), None, 7),         # small cells, one wave each, chunks across row ends
+])
+def test_scores_of_cells_of_every_size(shape, resolution, tile):
+    """Cells on both sides of the large-cell rule against the oracle's sequential totals, bit for bit,
+    continuing totals that are not zero."""
+    regions = (5, 3)
+    grid, decoder = _model(6, regions[0] * regions[1])
+    image = synth.image(8, shape[1], shape[0]).reshape(-1, 3)
+    target = torch.from_numpy(image).cuda()
+    n = shape[0] * shape[1]
+    _, scores = score_image(grid, decoder.half, target, shape, regions, resolution=resolution, tile=tile)
+    prediction = reconstruct(grid, decoder.half, shape, regions, 0, n).cpu().numpy()
+    expected = oracle.residual(prediction, image, shape[1], scores.resolution, scores.xb.cpu().numpy(),
+                               scores.yb.cpu().numpy())
+    assert np.array_equal(scores.totals.cpu().numpy().view(np.uint64), expected.view(np.uint64))
+
+
+@pytest.mark.parametrize('encoding', [
+    dict(n_levels=16, base_resolution=3, log2_hashmap_size=15, per_level_scale=1.9, n_features_per_level=2),
+    dict(n_levels=16, base_resolution=16, log2_hashmap_size=9, per_level_scale=1.38, n_features_per_level=2),
+    dict(n_levels=16, base_resolution=8, log2_hashmap_size=20, per_level_scale=1.2, n_features_per_level=2),   # all dense
+    dict(n_levels=16, base_resolution=40, log2_hashmap_size=6, per_level_scale=2.0, n_features_per_level=2),   # all hashed, past 2^12 cells
+])
+def test_reconstruction_encode_over_level_kinds(encoding):
+    """The reconstruction's own encode against odie_grid_forward on the routed coordinates: dense,
+    hashed and mixed lane steps, power-of-two and other level sizes, coordinates of exactly 0 and 1."""
+    shape, regions = (77, 201), (4, 3)
+    grid = ExpertGrid(encoding, regions[0] * regions[1])
+    grid.table.copy_(torch.from_numpy(synth.table(9, grid.table.numel(), -1.0, 1.0, name='kinds')).half())
+    decoder = Decoder(seed=9)
+    n = shape[0] * shape[1]
+    features = torch.empty((n, 32), dtype=torch.float16, device='cuda')
+    output = torch.empty((n, 16), dtype=torch.float16, device='cuda')
+    reconstruct(grid, decoder.half, shape, regions, 0, n, features=features, output=output)
+    want_features, want_output = _composed(grid, decoder, shape, regions, 0, n)
+    assert np.array_equal(_bits(features), _bits(want_features))
+    assert np.array_equal(_bits(output), _bits(want_output))
+
+
+def test_infinite_predictions_keep_their_scores():
+    """A decoder that overflows fp16 scores infinite and NaN totals exactly as score_chunk does."""
+    shape, regions = (64, 96), (2, 2)
+    grid, decoder = _model(10, 4)
+    decoder.params.mul_(3000.0)
+    decoder.sync_weights()
+    image = torch.from_numpy(synth.image(3, shape[1], shape[0]).reshape(-1, 3)).cuda()
+    n = shape[0] * shape[1]
+    prediction = reconstruct(grid, decoder.half, shape, regions, 0, n)
+    assert not bool(torch.isfinite(prediction).all())
+    streamed = DeviceScores(shape, resolution=4)
+    streamed.add(prediction, image, 0)
+    expected = oracle.residual(prediction.cpu().numpy(), image.cpu().numpy(), shape[1], 4, streamed.xb.cpu().numpy(),
+                               streamed.yb.cpu().numpy())
+    got = streamed.totals.cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(expected)) and np.array_equal(np.isinf(got), np.isinf(expected))
+    finite = np.isfinite(expected)
+    assert np.array_equal(got[finite], expected[finite])
