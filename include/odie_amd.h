@@ -163,7 +163,8 @@ int odie_grid_backward_adam_planes_handoff(const float* coords, int64_t n, const
  * "owner_lds_bytes", "paired_loads" (the forward's 16-byte corner-pair loads: 0 off, 1 on,
  * 2 (default) when one expert's fp16 table is larger than 1 MB), "forward_lds_bytes", "packed_owner" (1: the packed-plane
  * backward computes each slice of the gradient in one workgroup, 0 (default): global atomics),
- * "packed_splits" (0 = automatic), "route_part" (the routes' smallest sub-chunk of ids, a power
+ * "packed_splits" (0 = automatic), "packed_tiles" (1, the default: packed backwards given scratch sum
+ * by spatial tiles; 0: as without scratch), "route_part" (the routes' smallest sub-chunk of ids, a power
  * of two within 64..65536, default 512; size route workspaces after setting it),
  * "route_one_scan" (1, the default: the routes scan their counts in one launch when they have at
  * most 1024 segments of 1024 counts; 0: the reduce and apply launches).  Results do
@@ -191,6 +192,18 @@ int odie_packed_backward(const float* coords, int64_t n, const uint16_t* upstrea
                          const int32_t* descriptors, int levels, const uint64_t* node_bitmap,
                          const int32_t* node_prefix, const uint8_t* bitmap, float* gradient,
                          int64_t parameter_count, uint64_t stream);
+
+/* odie_packed_backward with caller-owned device scratch of odie_packed_backward_workspace(n, up_width)
+ * bytes (0 for batches that take none; -1 for arguments odie_packed_backward refuses): the
+ * coordinates are sorted into spatial tiles and each plane node's sum is formed in LDS, each
+ * contribution the fp32 product w * u rounded to 2^-30 of its column's largest finite |u| (fp32 sums
+ * where a contribution is infinite or NaN).  Calls with their own scratch may overlap.  No
+ * counterpart in the reference. */
+int64_t odie_packed_backward_workspace(int64_t n, int up_width);
+int odie_packed_backward_scratch(const float* coords, int64_t n, const uint16_t* upstream, int up_width,
+                                 const int32_t* descriptors, int levels, const uint64_t* node_bitmap,
+                                 const int32_t* node_prefix, const uint8_t* bitmap, float* gradient,
+                                 int64_t parameter_count, void* scratch, int64_t scratch_bytes, uint64_t stream);
 
 /* ---------------------------------------------------------------------------------------
  * Expert routing and compaction.  No counterpart in the reference (its "routing" is a soft

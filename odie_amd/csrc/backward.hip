@@ -1442,6 +1442,460 @@ __global__ __launch_bounds__(256) void packed_reduce_kernel(PackedOwnerArgs a) {
     }
 }
 
+// ---------------------------------------------------------------------------------------
+// Packed xy planes by spatial tiles: the backward of batches with caller-owned scratch.
+//
+// Bound by: scattered straight into memory, every contribution past the coarse planes is a global
+// fp32 atomic, about 20 G/s whatever the footprint (20 levels, 100,003 coordinates: 8 M of them,
+// 410 us).  Here they are added in LDS (64-bit fixed point at 2 T/s, as in the owner pass) and a
+// node's sum is stored once:
+//  1. packed_bin_kernel: the coordinates counted into 32 x 32 bins of the unit square per part of
+//     the batch; every upstream column's largest finite |u|; the gradient cleared;
+//  2. packed_place_kernel: the coordinates sorted by bin (their order within a bin is free: the
+//     sums are of integers);
+//  3. packed_tile_kernel: a workgroup per (level, tile of 2 x 2 bins).  At a level of R >= 49 it
+//     owns the nodes of columns first_node(2 tx) .. first_node(2 tx + 2) and the same rows, which
+//     only coordinates of its own bins and of the bin row and column before them reach (two before
+//     where a bin may span fewer than two nodes: a bin's cells end at the next bin's first node,
+//     their corners one further).  It adds their corners in LDS and stores the nodes that are not
+//     zero.  Coarser
+//     levels (at most 48^2 nodes) are summed by up to 32 workgroups over parts of the batch and added
+//     with atomics.
+// Corners that wrap -- past a row's end to the next row's first node, past the last row to the
+// first -- go to memory with atomics from the coordinate's own tile, as do the sums of the nodes
+// they can reach (column 0, row 0).
+// Scale: each column's contributions times 2^S rounded to 32 bits, S from the column's largest finite
+// |u| (quantum 2^-30 of it).  A workgroup that meets a contribution the scale does not cover (an
+// infinite or NaN upstream, weights off [0, 1] from coordinates beyond 2^31 cells or NaN) starts
+// again with fp32 sums, which carry them as the atomics do.
+// Measured (whole backward, us, atomics -> tiles): 20 levels of 954,016 parameters 1024 coordinates
+// 108 -> 44, 131,072 491 -> 94 (334 -> 90 in spatial order), 2^20 3393 -> 469; 8 levels 44 -> 26, 198 -> 53,
+// 1395 -> 242.  Of the 100,003-coordinate backward 7 us are the binning, 8 the placing and the
+// clearing's share, 75 the tiles: chains of dependent loads (list entry, cell bit and upstream; then the
+// node's prefix and word) in two workgroups of eight waves per CU, whose LDS a 1020-cell level fills.
+// Workgroups of 1024 threads: 20 us slower (one per CU at these registers).
+// ---------------------------------------------------------------------------------------
+constexpr int kBinSide = 32, kTileBins = kBinSide * kBinSide;
+constexpr int kTileSide = kBinSide / 2, kTiles = kTileSide * kTileSide;
+constexpr int kFineResolution = 49;                 // two bins span (R - 1) / 16 >= 3 cells: two nodes or more
+constexpr int kWideResolution = 97;                 // ... and so does one bin
+constexpr int kTileLdsValues = 48 * 48 * 4;         // the largest coarse level with F = 4: 72 KB
+constexpr int kBinBlock = 1024, kTileBlock = 512;
+constexpr int kMaxBinParts = 64, kMaxPeakBlocks = 128;
+constexpr int kTileFlush = 3;                       // nodes a thread stores with their row lookups in flight together
+
+struct PackedTileArgs {
+    const float* coords;
+    const uint16_t* upstream;     // fp16 [n][width]
+    const int32_t* desc;
+    const uint64_t* node_bitmap;
+    const int32_t* prefix;
+    const uint8_t* bitmap;
+    float* gradient;
+    int64_t n;
+    int64_t params;
+    int levels;
+    int width;
+    int parts;                    // parts of the batch counted apart (and placed by a block each)
+    int peak_blocks;
+    int fill_blocks;              // 0: the caller has cleared the gradient
+    int splits;                   // workgroups per coarse level
+    uint32_t* counts;             // [parts][kTileBins]
+    uint32_t* peaks;              // [peak_blocks][width]
+    uint32_t* bounds;             // [width]
+    uint32_t* starts;             // [kTileBins + 1]
+    float4* sorted;               // [n]: the coordinates sorted by bin: x, y and the index's bits
+};
+
+__device__ inline int bin_of(float v) {   // NaN: bin 0, as its cell is 0
+    const int b = static_cast<int>(fminf(fmaxf(v * static_cast<float>(kBinSide), 0.0f), static_cast<float>(kBinSide)));
+    return b < kBinSide ? b : kBinSide - 1;
+}
+__device__ inline int bin_of(float2 p) { return bin_of(p.y) * kBinSide + bin_of(p.x); }
+
+__device__ inline int64_t part_begin(const PackedTileArgs& a, int part) {
+    const int64_t share = (a.n + a.parts - 1) / a.parts;
+    return share * part < a.n ? share * part : a.n;
+}
+
+__global__ __launch_bounds__(kBinBlock) void packed_bin_kernel(PackedTileArgs a) {
+    __shared__ uint32_t shared[kTileBins];
+    shared[threadIdx.x] = 0;
+    __syncthreads();
+    int block = blockIdx.x;
+    if (block < a.parts) {
+        const int64_t end = part_begin(a, block + 1);
+        for (int64_t i = part_begin(a, block) + threadIdx.x; i < end; i += kBinBlock)
+            atomicAdd(shared + bin_of(reinterpret_cast<const float2*>(a.coords)[i]), 1u);
+        __syncthreads();
+        a.counts[block * kTileBins + threadIdx.x] = shared[threadIdx.x];
+        return;
+    }
+    block -= a.parts;
+    if (block < a.peak_blocks) {
+        // thread t takes column t % width of every (kBinBlock / width)-th row, eight loads in flight
+        const int per = kBinBlock / a.width, column = threadIdx.x % a.width, first = threadIdx.x / a.width;
+        const int64_t stride = static_cast<int64_t>(a.peak_blocks) * per;
+        uint32_t mine = 0;
+        if (first < per) {
+            for (int64_t row = static_cast<int64_t>(block) * per + first; row < a.n; row += 8 * stride) {
+                uint32_t m[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int64_t at = row + j * stride < a.n ? row + j * stride : row;
+                    m[j] = a.upstream[at * a.width + column] & 0x7fffu;
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j) mine = max(mine, m[j] < 0x7c00u ? m[j] : 0u);
+            }
+        }
+        if (mine) atomicMax(shared + column, mine);
+        __syncthreads();
+        if (static_cast<int>(threadIdx.x) < a.width) a.peaks[block * a.width + threadIdx.x] = shared[threadIdx.x];
+        return;
+    }
+    block -= a.peak_blocks;
+    for (int64_t j = static_cast<int64_t>(block) * kBinBlock + threadIdx.x; j < a.params;
+         j += static_cast<int64_t>(a.fill_blocks) * kBinBlock)
+        a.gradient[j] = 0.0f;
+}
+
+__global__ __launch_bounds__(kBinBlock) void packed_place_kernel(PackedTileArgs a) {
+    __shared__ uint32_t cursor[kTileBins];
+    if (static_cast<int>(blockIdx.x) == a.parts) {
+        // the blocks' peaks, eight threads a column
+        cursor[threadIdx.x] = 0;
+        __syncthreads();
+        const int column = threadIdx.x % 128, first = threadIdx.x / 128;
+        if (column < a.width) {
+            uint32_t most = 0;
+#pragma unroll 8
+            for (int b = first; b < a.peak_blocks; b += 8) most = max(most, a.peaks[b * a.width + column]);
+            atomicMax(cursor + column, most);
+        }
+        __syncthreads();
+        if (static_cast<int>(threadIdx.x) < a.width) a.bounds[threadIdx.x] = cursor[threadIdx.x];
+        return;
+    }
+    // this thread's bin: how many coordinates it holds, and how many in the parts before this one
+    const int part = blockIdx.x, bin = threadIdx.x;
+    uint32_t total = 0, before = 0;
+#pragma unroll 8
+    for (int q = 0; q < a.parts; ++q) {
+        const uint32_t count = a.counts[q * kTileBins + bin];
+        total += count;
+        before += q < part ? count : 0u;
+    }
+    // exclusive scan of the totals over the block: within waves by shuffles, then over the 16 waves
+    const int lane = bin % 64, wave = bin / 64;
+    uint32_t run = total;
+    for (int step = 1; step < 64; step <<= 1) {
+        const uint32_t below = __shfl_up(run, step);
+        run += lane >= step ? below : 0u;
+    }
+    if (lane == 63) cursor[wave] = run;
+    __syncthreads();
+    uint32_t earlier = 0;
+#pragma unroll
+    for (int q = 0; q < kBinBlock / 64; ++q) earlier += q < wave ? cursor[q] : 0u;
+    const uint32_t start = earlier + run - total;
+    __syncthreads();
+    cursor[bin] = start + before;
+    if (part == 0) {
+        a.starts[bin] = start;
+        if (bin == kTileBins - 1) a.starts[kTileBins] = start + total;
+    }
+    __syncthreads();
+    const int64_t end = part_begin(a, part + 1);
+    for (int64_t i = part_begin(a, part) + threadIdx.x; i < end; i += kBinBlock) {
+        const float2 p = reinterpret_cast<const float2*>(a.coords)[i];
+        const uint32_t at = atomicAdd(cursor + bin_of(p), 1u);
+        a.sorted[at] = make_float4(p.x, p.y, __uint_as_float(static_cast<uint32_t>(i)), 0.0f);
+    }
+}
+
+// First node column (or row) of bin b at resolution r: the cell of the bin's lower edge, by the
+// cells' own arithmetic, so every coordinate of the bin has a cell at or after it.
+__device__ inline int first_node(int b, int r) {
+    return b >= kBinSide ? r : static_cast<int>(floorf(__builtin_fmaf(static_cast<float>(r - 1),
+                                                                      static_cast<float>(b) / kBinSide, 0.5f)));
+}
+
+// One coordinate at one level: its cell (clamped as plane_geometry clamps it) and corner weights.
+struct TileCorner {
+    int ix, iy;
+    float w[4];
+    bool regular;   // weights within [0, 1]
+    __device__ __forceinline__ TileCorner(float2 p, int r) {
+        const float px = __builtin_fmaf(static_cast<float>(r - 1), p.x, 0.5f);
+        const float py = __builtin_fmaf(static_cast<float>(r - 1), p.y, 0.5f);
+        ix = static_cast<int>(floorf(px));
+        iy = static_cast<int>(floorf(py));
+        const float fx = px - static_cast<float>(ix), fy = py - static_cast<float>(iy);
+        regular = fx >= 0.0f && fx <= 1.0f && fy >= 0.0f && fy <= 1.0f;
+        ix = ix < 0 ? 0 : (ix > r - 1 ? r - 1 : ix);
+        iy = iy < 0 ? 0 : (iy > r - 1 ? r - 1 : iy);
+        w[0] = (1.0f - fx) * (1.0f - fy);
+        w[1] = fx * (1.0f - fy);
+        w[2] = (1.0f - fx) * fy;
+        w[3] = fx * fy;
+    }
+};
+
+// Row of a stored node and the parameter of its feature c.
+__device__ inline int node_row(const PackedTileArgs& a, const int32_t* d, int node) {
+    if (d[7]) return node;
+    const int word = d[3] + (node >> 6);
+    return a.prefix[word] + __popcll(a.node_bitmap[word] & ((uint64_t{1} << (node & 63)) - uint64_t{1}));
+}
+
+template <int F> struct TileLevel {
+    const PackedTileArgs& a;
+    const int32_t* d;
+    int r, points, column;
+    int64_t cells;          // byte offset of the level's cell bits
+    int used;               // features with an upstream column
+    int32_t shift[F];
+    float scale[F], peak[F];
+
+    __device__ __forceinline__ TileLevel(const PackedTileArgs& args, const int32_t* desc)
+        : a(args), d(desc), r(desc[0]), points(desc[1]), column(desc[6]), cells(desc[4]) {
+        used = 0;
+#pragma unroll
+        for (int c = 0; c < F; ++c) {
+            const bool real = column + c < a.width;
+            used += real;
+            peak[c] = real ? __half2float(bits_to_half(static_cast<uint16_t>(a.bounds[column + c]))) : 0.0f;
+            shift[c] = column_shift(__float_as_uint(peak[c]), a.n);
+            scale[c] = shift_scale(shift[c]);
+        }
+    }
+    __device__ __forceinline__ bool visible(int cell) const { return (a.bitmap[cells + (cell >> 3)] >> (cell & 7)) & 1; }
+    // The upstream values of row i; false when one is not within its column's finite peak.
+    __device__ __forceinline__ bool load(int64_t i, float u[F]) const {
+        const uint16_t* row = a.upstream + i * a.width + column;
+        bool regular = true;
+#pragma unroll
+        for (int c = 0; c < F; ++c) {
+            u[c] = c < used ? __half2float(bits_to_half(row[c])) : 0.0f;
+            regular = regular && fabsf(u[c]) <= peak[c];
+        }
+        return regular;
+    }
+    // Adds w * u of one corner to the F accumulators from slot `at`.
+    __device__ __forceinline__ void add(unsigned long long* acc, bool exact, int at, float w, const float u[F]) const {
+#pragma unroll
+        for (int c = 0; c < F; ++c) {
+            if (u[c] == 0.0f) continue;
+            if (exact) {
+                const int32_t q = round_to_int(w * u[c] * scale[c]);
+                atomicAdd(acc + at * F + c, static_cast<unsigned long long>(static_cast<long long>(q)));
+            } else {
+                atomicAdd(reinterpret_cast<float*>(acc) + at * F + c, w * u[c]);
+            }
+        }
+    }
+    __device__ __forceinline__ float value(const unsigned long long* acc, bool exact, int slot, int c) const {
+        return exact ? unscaled(static_cast<long long>(acc[slot]), shift[c]) : reinterpret_cast<const float*>(acc)[slot];
+    }
+    __device__ __forceinline__ float* parameter(int row, int c) const { return a.gradient + packed_at(d, a.params, row, c); }
+};
+
+// A part of the batch at a coarse level: every node in LDS, the sums added to the gradient.
+template <int F>
+__device__ __forceinline__ void coarse_level(const TileLevel<F>& level, int split, unsigned long long* acc, int& irregular) {
+    const PackedTileArgs& a = level.a;
+    const int64_t share = (a.n + a.splits - 1) / a.splits;
+    const int64_t b0 = share * split, b1 = b0 + share < a.n ? b0 + share : a.n;
+    if (b0 >= b1) return;
+    const int slots = level.points * F;
+    for (int attempt = 0; attempt < 2; ++attempt) {
+        const bool exact = attempt == 0;
+        for (int j = threadIdx.x; j < slots; j += kTileBlock) acc[j] = 0;
+        if (threadIdx.x == 0) irregular = 0;
+        __syncthreads();
+        // a wave's lanes take coordinates `rows` apart: a batch in spatial order would otherwise put them
+        // on one node, and LDS adds to one address serialize
+        const int rows = static_cast<int>((b1 - b0 + 63) / 64);
+        for (int k = threadIdx.x / 64; k < rows; k += kTileBlock / 64) {
+            const int64_t i = b0 + static_cast<int64_t>(threadIdx.x % 64) * rows + k;
+            if (i >= b1) continue;
+            const TileCorner at(reinterpret_cast<const float2*>(a.coords)[i], level.r);
+            const int cell = at.ix + at.iy * level.r;
+            if (!level.visible(cell)) continue;
+            float u[F];
+            const bool regular = level.load(i, u) && at.regular;
+            if (exact && !regular) {
+                irregular = 1;
+                continue;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int node = cell + (k & 1) + (k >> 1) * level.r;
+                level.add(acc, exact, node < level.points ? node : node - level.points, at.w[k], u);
+            }
+        }
+        __syncthreads();
+        if (!exact || !irregular) {
+            for (int node = threadIdx.x; node < level.points; node += kTileBlock) {
+                float v[F];
+                bool any = false;
+#pragma unroll
+                for (int c = 0; c < F; ++c) {
+                    v[c] = level.value(acc, exact, node * F + c, c);
+                    any = any || v[c] != 0.0f;
+                }
+                if (!any) continue;
+                const int row = node_row(a, level.d, node);
+#pragma unroll
+                for (int c = 0; c < F; ++c)
+                    if (v[c] != 0.0f) atomicAdd(level.parameter(row, c), v[c]);
+            }
+            return;
+        }
+        __syncthreads();
+    }
+}
+
+// The nodes [x0, x1) x [y0, y1) of a tile at a fine level, in pieces that fit LDS.
+template <int F>
+__device__ __forceinline__ void fine_tile(const TileLevel<F>& level, int tx, int ty, unsigned long long* acc, int& irregular) {
+    const PackedTileArgs& a = level.a;
+    const int r = level.r;
+    const int x0 = first_node(2 * tx, r), x1 = first_node(2 * tx + 2, r);
+    const int y0 = first_node(2 * ty, r), y1 = first_node(2 * ty + 2, r);
+    // the list runs of the bins that reach them: bins 2tx-back .. 2tx+1 of rows 2ty-back .. 2ty+1
+    const int back = r < kWideResolution ? 2 : 1;
+    const int bx = max(2 * tx - back, 0);
+    int64_t from[4], upto[4];   // first list position and end of the concatenation, per bin row
+    int64_t total = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int by = 2 * ty - back + q;
+        const bool row = by >= 0 && by < 2 * ty + 2;
+        from[q] = row ? a.starts[by * kBinSide + bx] : 0;
+        total += row ? a.starts[by * kBinSide + 2 * tx + 2] - from[q] : 0;
+        upto[q] = total;
+    }
+    if (total == 0) return;
+    const int cap = kTileLdsValues / F;
+    const int piece_x = min(x1 - x0, cap), piece_y = min(y1 - y0, max(1, cap / piece_x));
+    bool first = true;
+    for (int py = y0; py < y1; py += piece_y)
+        for (int px = x0; px < x1; px += piece_x) {
+            const int nx = min(piece_x, x1 - px), ny = min(piece_y, y1 - py);
+            for (int attempt = 0; attempt < 2; ++attempt) {
+                const bool exact = attempt == 0;
+                __syncthreads();
+                for (int j = threadIdx.x; j < nx * ny * F; j += kTileBlock) acc[j] = 0;
+                if (threadIdx.x == 0) irregular = 0;
+                __syncthreads();
+                for (int64_t j = threadIdx.x; j < total; j += kTileBlock) {
+                    int64_t pos = from[0] + j;
+                    pos = j >= upto[0] ? from[1] + j - upto[0] : pos;
+                    pos = j >= upto[1] ? from[2] + j - upto[1] : pos;
+                    pos = j >= upto[2] ? from[3] + j - upto[2] : pos;
+                    const float4 entry = a.sorted[pos];
+                    const float2 p = make_float2(entry.x, entry.y);
+                    const TileCorner at(p, r);
+                    const int lx = at.ix - px, ly = at.iy - py;   // inside: corners lx, lx + 1 in [0, nx)
+                    const bool inside = lx >= -1 && lx < nx && ly >= -1 && ly < ny;
+                    const bool wraps = exact && first && (at.ix == r - 1 || at.iy == r - 1) &&
+                                       (bin_of(p.x) >> 1) == tx && (bin_of(p.y) >> 1) == ty;
+                    if (!inside && !wraps) continue;
+                    const int cell = at.ix + at.iy * r;
+                    float u[F];   // loaded beside the cell's bit, not after it
+                    const bool seen = level.visible(cell);
+                    const bool regular = level.load(__float_as_uint(entry.z), u) && at.regular;
+                    if (!seen) continue;
+                    if (inside) {
+                        if (exact && !regular) {
+                            irregular = 1;
+                        } else {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) {
+                                const int cx = lx + (k & 1), cy = ly + (k >> 1);
+                                const bool here = cx >= 0 && cx < nx && cy >= 0 && cy < ny;
+                                if (here) level.add(acc, exact, cy * nx + cx, at.w[k], u);
+                            }
+                        }
+                    }
+                    if (wraps) {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            if (at.ix + (k & 1) < r && at.iy + (k >> 1) < r) continue;
+                            const int node = (cell + (k & 1) + (k >> 1) * r) % level.points;
+                            const int row = node_row(a, level.d, node);
+#pragma unroll
+                            for (int c = 0; c < F; ++c)
+                                if (u[c] != 0.0f) atomicAdd(level.parameter(row, c), at.w[k] * u[c]);
+                        }
+                    }
+                }
+                __syncthreads();
+                if (exact && irregular) continue;
+                for (int j0 = threadIdx.x; j0 < nx * ny; j0 += kTileFlush * kTileBlock) {
+                    float v[kTileFlush][F];
+                    int row[kTileFlush], node[kTileFlush];
+#pragma unroll
+                    for (int q = 0; q < kTileFlush; ++q) {
+                        const int j = j0 + q * kTileBlock;
+                        bool any = false;
+#pragma unroll
+                        for (int c = 0; c < F; ++c) {
+                            v[q][c] = j < nx * ny ? level.value(acc, exact, j * F + c, c) : 0.0f;
+                            any = any || v[q][c] != 0.0f;
+                        }
+                        node[q] = any ? px + j % nx + (py + j / nx) * r : -1;
+                        row[q] = any ? node_row(a, level.d, node[q]) : 0;
+                    }
+#pragma unroll
+                    for (int q = 0; q < kTileFlush; ++q) {
+                        if (node[q] < 0) continue;
+                        const bool shared_node = node[q] < r || node[q] % r == 0;
+#pragma unroll
+                        for (int c = 0; c < F; ++c) {
+                            if (shared_node) {
+                                if (v[q][c] != 0.0f) atomicAdd(level.parameter(row[q], c), v[q][c]);
+                            } else {
+                                *level.parameter(row[q], c) = v[q][c];
+                            }
+                        }
+                    }
+                }
+                break;
+            }
+            first = false;
+        }
+}
+
+template <int F>
+__device__ __forceinline__ void tile_level(const PackedTileArgs& a, const int32_t* d, int slot, unsigned long long* acc,
+                                  int& irregular) {
+    const TileLevel<F> level(a, d);
+    if (level.used == 0) return;
+    if (level.r < kFineResolution) {
+        if (slot < a.splits) coarse_level(level, slot, acc, irregular);
+        return;
+    }
+    // consecutive tiles on one XCD (a block's XCD is its index mod 8), so that they share its L2
+    const int tile = (slot % kXcds) * (kTiles / kXcds) + slot / kXcds;
+    fine_tile(level, tile % kTileSide, tile / kTileSide, acc, irregular);
+}
+
+__global__ __launch_bounds__(kTileBlock) void packed_tile_kernel(PackedTileArgs a) {
+    extern __shared__ unsigned long long acc[];
+    __shared__ int irregular;
+    const int slot = blockIdx.x % kTiles;
+    const int32_t* d = a.desc + 8 * (blockIdx.x / kTiles);
+    switch (d[5]) {
+        case 1: tile_level<1>(a, d, slot, acc, irregular); break;
+        case 2: tile_level<2>(a, d, slot, acc, irregular); break;
+        case 4: tile_level<4>(a, d, slot, acc, irregular); break;
+        default: break;
+    }
+}
+
 template <typename Kernel>
 int allow_lds(Kernel kernel, size_t bytes) {
     const hipError_t status = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -1862,6 +2316,61 @@ int launch_band_lists(const OwnerLaunch& in, const HandoffPlan& plan, uint8_t* h
                             reinterpret_cast<int32_t*>(handoff + plan.list_at),
                             reinterpret_cast<float2*>(handoff + plan.sorted_at),
                             reinterpret_cast<int32_t*>(handoff + plan.ordered_at));
+}
+
+namespace {
+
+struct TileLayout { size_t peaks, bounds, starts, sorted, total; int parts, peak_blocks; };
+
+TileLayout tile_layout(int64_t n, int width) {
+    const auto align = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    TileLayout l{};
+    l.parts = static_cast<int>(std::min<int64_t>(std::max<int64_t>(n / 2048, 1), kMaxBinParts));
+    l.peak_blocks = static_cast<int>(std::min<int64_t>(std::max<int64_t>(n / 512, 1), kMaxPeakBlocks));
+    l.peaks = align(sizeof(uint32_t) * l.parts * kTileBins);
+    l.bounds = l.peaks + align(sizeof(uint32_t) * l.peak_blocks * width);
+    l.starts = l.bounds + align(sizeof(uint32_t) * width);
+    l.sorted = l.starts + align(sizeof(uint32_t) * (kTileBins + 1));
+    l.total = l.sorted + align(sizeof(float4) * n);
+    return l;
+}
+
+}  // namespace
+
+int64_t packed_tile_workspace(int64_t n, int width) { return static_cast<int64_t>(tile_layout(n, width).total); }
+
+int launch_packed_tiles(const float* coords, int64_t n, const uint16_t* upstream, int width, const int32_t* desc,
+                        int levels, const uint64_t* node_bitmap, const int32_t* node_prefix, const uint8_t* bitmap,
+                        float* gradient, int64_t params, bool zeroed, void* workspace, hipStream_t stream) {
+    const TileLayout l = tile_layout(n, width);
+    char* space = static_cast<char*>(workspace);
+    PackedTileArgs a{};
+    a.coords = coords;
+    a.upstream = upstream;
+    a.desc = desc;
+    a.node_bitmap = node_bitmap;
+    a.prefix = node_prefix;
+    a.bitmap = bitmap;
+    a.gradient = gradient;
+    a.n = n;
+    a.params = params;
+    a.levels = levels;
+    a.width = width;
+    a.parts = l.parts;
+    a.peak_blocks = l.peak_blocks;
+    a.fill_blocks = zeroed ? 0 : static_cast<int>(std::min<int64_t>((params + kBinBlock - 1) / kBinBlock, kCus));
+    a.splits = static_cast<int>(std::min<int64_t>(std::max<int64_t>(n / 2048, 1), 32));
+    a.counts = reinterpret_cast<uint32_t*>(space);
+    a.peaks = reinterpret_cast<uint32_t*>(space + l.peaks);
+    a.bounds = reinterpret_cast<uint32_t*>(space + l.bounds);
+    a.starts = reinterpret_cast<uint32_t*>(space + l.starts);
+    a.sorted = reinterpret_cast<float4*>(space + l.sorted);
+    constexpr size_t shmem = sizeof(unsigned long long) * kTileLdsValues;
+    if (allow_lds(packed_tile_kernel, shmem)) return -1;
+    packed_bin_kernel<<<static_cast<uint32_t>(a.parts + a.peak_blocks + a.fill_blocks), kBinBlock, 0, stream>>>(a);
+    packed_place_kernel<<<static_cast<uint32_t>(a.parts + 1), kBinBlock, 0, stream>>>(a);
+    packed_tile_kernel<<<static_cast<uint32_t>(levels * kTiles), kTileBlock, shmem, stream>>>(a);
+    return check_launch("odie_packed_backward");
 }
 
 int launch_packed_owner(const float* coords, int64_t n, const uint16_t* upstream, int width, const int32_t* desc,

@@ -240,6 +240,13 @@ int launch_packed_owner(const float* coords, int64_t n, const uint16_t* upstream
                         int levels, const uint64_t* node_bitmap, const int32_t* node_prefix, const uint8_t* bitmap,
                         float* gradient, int64_t params, int64_t lds_bytes, int64_t splits, hipStream_t stream);
 
+// The same gradient by spatial tiles (backward.hip), with scratch of packed_tile_workspace bytes;
+// zeroed: the caller has cleared the gradient.  width <= 128.
+int64_t packed_tile_workspace(int64_t n, int width);
+int launch_packed_tiles(const float* coords, int64_t n, const uint16_t* upstream, int width, const int32_t* desc,
+                        int levels, const uint64_t* node_bitmap, const int32_t* node_prefix, const uint8_t* bitmap,
+                        float* gradient, int64_t params, bool zeroed, void* workspace, hipStream_t stream);
+
 // odie_grid_backward_adam with the optimizer step already formed (adam.h), so that callers
 // can set fields the C ABI does not expose (the fp16 gradient store).
 int grid_backward_adam_internal(const float* coords, int64_t n, const int32_t* offsets, int experts,
@@ -260,11 +267,13 @@ int grid_backward_adam_planes_internal(const float* coords, int64_t n, const int
 // pairs: the caller guarantees 2 features at output offset 2l for every level but the last,
 // which has 1 or 2 (the pairs kernel applies when the row is a multiple of 16 columns).
 // odie_packed_backward on `s`; zeroed: the caller has already cleared `gradient` (the atomics
-// path then adds into it without clearing it first).
+// and tile paths then add into it without clearing it first).  scratch: odie_packed_backward_workspace
+// bytes for the tile path, or null.
 int packed_backward_internal(const float* coords, int64_t n, const uint16_t* upstream, int up_width,
                              const int32_t* descriptors, int levels, const uint64_t* node_bitmap,
                              const int32_t* node_prefix, const uint8_t* bitmap, float* gradient,
-                             int64_t parameter_count, hipStream_t s, bool zeroed);
+                             int64_t parameter_count, hipStream_t s, bool zeroed, void* scratch = nullptr,
+                             int64_t scratch_bytes = 0);
 
 int packed_forward_internal(const float* coords, int64_t n, const float* grid, int64_t parameter_count,
                             const int32_t* descriptors, int levels, const uint64_t* node_bitmap,

@@ -296,6 +296,7 @@ struct Runtime {
     DeviceBuffer<uint16_t> grid_half;
     // work buffers, B = 65536 rows
     DeviceBuffer<float> xy, target, squares, sigmoid, grid_grad;
+    DeviceBuffer<uint8_t> packed_scratch;
     DeviceBuffer<uint32_t> colors;
     DeviceBuffer<uint16_t> raw, weighted, dz, upstream, output;
     DeviceBuffer<uint8_t> vis;
@@ -412,6 +413,7 @@ Runtime::Runtime(const Json& j)
     vis.allocate(static_cast<size_t>(levels) * kBatch);
     flag.allocate(1);
     grid_grad.allocate(total);
+    if (!hash) packed_scratch.allocate(packed_tile_workspace(kBatch, row));
     grid_grad.zero(stream);
     grid_adam.allocate(total, stream);
     decoder.reset(new Head(device_pointer<float>(j, "decoder"), decoder_params(row), stream));
@@ -542,7 +544,7 @@ void Runtime::step(const int64_t* ids, int n, bool update) {
                                 features[0], grid_grad.data, 1, s));
     } else {
         call(packed_backward_internal(xy.data, n, up, row, desc, levels, bits, prefix, cells, grid_grad.data, total,
-                                      stream, clear));
+                                      stream, clear, packed_scratch.data, packed_scratch.count));
         if (update)
             sets[pending++] = AdamSet{make_step(grid, nullptr, grid_adam, 1, grid_lr, 128.0f, grid_divisor),
                                       grid_grad.data, 0, total};

@@ -180,11 +180,14 @@ def packed_backward(coordinates, upstream, descriptors, node_bitmap, node_prefix
         raise ValueError('upstream must be CUDA contiguous FP16 NxF')
     upstream = upstream.contiguous()
     gradient = torch.empty(parameter_count, dtype=torch.float32, device=coordinates.device)
-    _lib.check(_lib.library().odie_packed_backward(
+    lib = _lib.library()
+    need = max(int(lib.odie_packed_backward_workspace(coordinates.shape[0], upstream.shape[1])), 0)
+    scratch = torch.empty(need, dtype=torch.uint8, device=coordinates.device) if need else None
+    _lib.check(lib.odie_packed_backward_scratch(
         coordinates.data_ptr(), coordinates.shape[0], upstream.data_ptr(), upstream.shape[1],
         descriptors.data_ptr(), descriptors.shape[0], _nonempty(node_bitmap).data_ptr(),
         _nonempty(node_prefix).data_ptr(), bitmap.data_ptr(), gradient.data_ptr(), parameter_count,
-        _lib.stream_of(coordinates)))
+        _lib.ptr(scratch), need, _lib.stream_of(coordinates)))
     return gradient
 
 
@@ -198,10 +201,13 @@ class PackedQuery(torch.autograd.Function):
         ctx.save_for_backward(coordinates, descriptors, node_bitmap, node_prefix, bitmap)
         ctx.param_count = grid.numel()
         ctx.mark_non_differentiable(visible)
+        ctx.set_materialize_grads(False)   # no zeros [N, L] for the visibility's absent gradient
         return features, visible
 
     @staticmethod
     def backward(ctx, feature_gradient, visibility_gradient):
+        if feature_gradient is None:
+            return (None,) * 7
         coordinates, descriptors, node_bitmap, node_prefix, bitmap = ctx.saved_tensors
         gradient = packed_backward(coordinates, feature_gradient.contiguous(), descriptors, node_bitmap,
                                    node_prefix, bitmap, ctx.param_count)

@@ -571,3 +571,129 @@ def test_owner_masks_are_bit_identical(log2, experts, n, outside):
     finally:
         _lib.set_tuning('banded', 2)
     assert torch.equal(masked.view(torch.int32), plain.view(torch.int32))
+
+
+# Levels on both sides of the tile pass's limits: coarse (48 and below), the smallest tiles, a level
+# whose tile fills LDS several times over (F = 4, 1200 cells a side), mixed features.
+TILE_PLANES = dict(resolutions=(8, 47, 48, 49, 50, 65, 130, 333, 1200), dims=(2, 4, 1, 2, 4, 1, 2, 2, 4), dense=4)
+
+
+def _without_tiles(layout, xy, up):
+    _lib.set_tuning('packed_tiles', 0)
+    try:
+        return _packed_gradient(layout, xy, up, packed_owner=0)
+    finally:
+        _lib.set_tuning('packed_tiles', 1)
+
+
+@pytest.mark.parametrize('n,width,spread', [(1024, 22, 'uniform'), (16384, 22, 'uniform'), (20001, 22, 'edges'),
+                                            (40000, 22, 'corner'),
+                                            (16385, 32, 'outside'), (70000, 20, 'stratified'), (16384, 2, 'uniform')])
+def test_packed_tiles_match_the_oracle_and_the_atomics(n, width, spread):
+    """The packed backward by spatial tiles: bins' edges, corners that wrap past a row or the plane,
+    coordinates off the unit square, every coordinate in one tile, fewer upstream columns than
+    features."""
+    layout = _packed_layout(21, **TILE_PLANES)
+    xy = synth.coordinates(21, n)
+    if spread == 'edges':       # bin edges, and the last half cell that wraps
+        grid = np.arange(33, dtype=np.float32) / 32
+        xy[:33 * 33] = np.stack(np.meshgrid(grid, grid), axis=-1).reshape(-1, 2)
+        xy[2000:6000, 0] = 1.0 - np.float32(1e-4) * xy[2000:6000, 0]
+        xy[6000:9000, 1] = 1.0 - np.float32(1e-4) * xy[6000:9000, 1]
+    elif spread == 'corner':
+        xy = xy * np.float32(0.03)
+    elif spread == 'outside':
+        xy = (xy * 3 - 1).astype(np.float32)
+    elif spread == 'stratified':
+        side = 256
+        j = np.arange(n)
+        xy = ((np.stack([j % side, j // side % side], axis=1) + xy) / side).astype(np.float32)
+    up = synth.upstream(21, n, width)
+    d_xy, d_up = torch.from_numpy(xy).cuda(), torch.from_numpy(up).cuda()
+    tiles = _packed_gradient(layout, d_xy, d_up, packed_owner=0)
+    atomics = _without_tiles(layout, d_xy, d_up)
+    if spread == 'outside':     # the oracle takes the unit square; the kernels clamp the cell
+        difference = (tiles.double() - atomics.double()).abs()
+        assert float(difference.max()) <= 1e-5 * float(atomics.abs().max())
+        return
+    host = {k: layout[k].numpy() for k in ('descriptors', 'node_bitmap', 'node_prefix', 'bitmap')}
+    columns = np.zeros((n, max(width, 22)), dtype=np.float16)   # a feature past the upstream's columns gets nothing
+    columns[:, :width] = up
+    bar = packed_bar(xy, columns, host, layout['params'])
+    check_gradient(tiles, bar, 'packed tiles, ' + spread)
+    check_gradient(atomics, bar, 'packed atomics, ' + spread)
+
+
+def test_packed_tiles_column_scales_and_zero_upstream():
+    """Columns 10^6 apart keep their own scale; an all-zero upstream clears the gradient."""
+    layout = _packed_layout(22, **TILE_PLANES)
+    n, width = 20000, 22
+    xy = synth.coordinates(22, n)
+    up = synth.upstream(22, n, width).astype(np.float32) * np.where(np.arange(width) % 2 == 0, 1e3, 1e-3)
+    up = up.astype(np.float16)
+    d_xy, d_up = torch.from_numpy(xy).cuda(), torch.from_numpy(up).cuda()
+    host = {k: layout[k].numpy() for k in ('descriptors', 'node_bitmap', 'node_prefix', 'bitmap')}
+    bar = packed_bar(xy, up, host, layout['params'])
+    got = _packed_gradient(layout, d_xy, d_up, packed_owner=0)
+    check_gradient(got, bar, 'packed tiles, columns 10^6 apart')
+    _check_relative(got, bar, 'packed tiles, columns 10^6 apart')
+    zero = _packed_gradient(layout, d_xy, torch.zeros_like(d_up), packed_owner=0)
+    assert not bool(zero.any())
+
+
+@pytest.mark.parametrize('case', ['inf', 'nan', 'nan_xy', 'far_xy', 'all_inf'])
+def test_packed_tiles_carry_infinities_and_nans_as_the_atomics_do(case):
+    layout = _packed_layout(23, **TILE_PLANES)
+    n, width = 20000, 22
+    xy = synth.coordinates(23, n)
+    up = synth.upstream(23, n, width)
+    if case == 'inf':
+        up[::997, 3] = np.inf
+        up[5::1999, 20] = -np.inf
+    elif case == 'nan':
+        up[::1013, :] = np.nan
+    elif case == 'nan_xy':
+        xy[::1511, 0] = np.nan
+        xy[7::1511, 1] = np.inf
+    elif case == 'far_xy':
+        xy[::1511, 0] = 1e12
+        xy[3::1511, 1] = -1e12
+    else:
+        up[:, 1] = np.inf
+    d_xy, d_up = torch.from_numpy(xy).cuda(), torch.from_numpy(up).cuda()
+    got, want = _packed_gradient(layout, d_xy, d_up, packed_owner=0), _without_tiles(layout, d_xy, d_up)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isinf(got) * got.sign(), torch.isinf(want) * want.sign())
+    fine = torch.isfinite(want)
+    assert bool(fine.any()) and bool(fine.all()) == (case == 'far_xy')   # there: huge finite weights
+    difference = (got[fine].double() - want[fine].double()).abs()
+    # sums of the same fp32 products in another order, beside a rounding to 2^-30 of the column's peak
+    assert float(difference.norm() / want[fine].double().norm()) < 1e-5
+
+
+def test_packed_backward_scratch_is_checked_and_ragged_streams_overlap():
+    """Too little scratch is refused; two streams with their own scratch do not disturb each other."""
+    layout = _packed_layout(24, **TILE_PLANES)
+    n, width = 30000, 22
+    d_xy = torch.from_numpy(synth.coordinates(24, n)).cuda()
+    d_up = torch.from_numpy(synth.upstream(24, n, width)).cuda()
+    lib = _lib.library()
+    need = lib.odie_packed_backward_workspace(n, width)
+    assert need > 0 and lib.odie_packed_backward_workspace(100, width) == 0
+    assert lib.odie_packed_backward_workspace(-1, width) == -1 and lib.odie_packed_backward_workspace(n, 1) == -1
+    want = _packed_gradient(layout, d_xy, d_up, packed_owner=0)
+    torch.cuda.synchronize()
+    streams, results = [torch.cuda.Stream() for _ in range(2)], []
+    for stream in streams:
+        with torch.cuda.stream(stream):
+            for _ in range(3):
+                results.append(_packed_gradient(layout, d_xy, d_up, packed_owner=0))
+    torch.cuda.synchronize()
+    for got in results:   # the wrapped corners' and coarse levels' fp32 atomics sum in any order
+        assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())
+    dev = {k: layout[k].cuda() for k in ('descriptors', 'node_bitmap', 'node_prefix', 'bitmap')}
+    scratch, gradient = torch.empty(need, dtype=torch.uint8, device='cuda'), torch.empty_like(want)
+    assert lib.odie_packed_backward_scratch(
+        d_xy.data_ptr(), n, d_up.data_ptr(), width, dev['descriptors'].data_ptr(), 9, dev['node_bitmap'].data_ptr(),
+        dev['node_prefix'].data_ptr(), dev['bitmap'].data_ptr(), gradient.data_ptr(), layout['params'],
+        scratch.data_ptr(), need - 1, 0) == -1
