@@ -183,6 +183,13 @@ int odie_packed_forward(const float* coords, int64_t n, const float* grid, int64
                         const int32_t* node_prefix, const uint8_t* bitmap, int width,
                         uint16_t* features, uint8_t* visibility, uint64_t stream);
 
+/* odie_packed_forward as the model's evaluation reads it (odie/model.py:266-279): the features of
+ * levels >= active times 0 and those levels not visible, columns past the last level 1.0. */
+int odie_packed_forward_rows(const float* coords, int64_t n, const float* grid, int64_t parameter_count,
+                             const int32_t* descriptors, int levels, const uint64_t* node_bitmap,
+                             const int32_t* node_prefix, const uint8_t* bitmap, int width, int active,
+                             uint16_t* features, uint8_t* visibility, uint64_t stream);
+
 /* gradient (fp32 [parameter_count]) is written whole, not accumulated, with fp32 atomics as
  * the reference does (summation order free).  With the tuning key "packed_owner" = 1 each slice
  * of it is summed by one workgroup in 64-bit fixed point instead: deterministic, each

@@ -40,6 +40,7 @@ SIGNATURES = {
                                                 _P, _I64, _U64], _I),
     'odie_grid_backward': ([_P, _I64, _P, _I, _P, _I, _I, _I64, _P, _I, _I, _P, _I, _U64], _I),
     'odie_packed_forward': ([_P, _I64, _P, _I64, _P, _I, _P, _P, _P, _I, _P, _P, _U64], _I),
+    'odie_packed_forward_rows': ([_P, _I64, _P, _I64, _P, _I, _P, _P, _P, _I, _I, _P, _P, _U64], _I),
     'odie_packed_backward': ([_P, _I64, _P, _I, _P, _I, _P, _P, _P, _P, _I64, _U64], _I),
     'odie_packed_backward_workspace': ([_I64, _I], _I64),
     'odie_packed_backward_scratch': ([_P, _I64, _P, _I, _P, _I, _P, _P, _P, _P, _I64, _P, _I64, _U64], _I),

@@ -492,161 +492,140 @@ struct PackedArgs {
     int width;
     int active;          // levels >= active are off (the native step's active prefix)
     uint16_t pad;        // fp16 bits written to columns past the last level
+    int zero_off;        // levels >= active are evaluated and multiplied by 0 (else 0 outright)
 };
 
 __device__ inline int64_t plane_param(const PackedArgs& a, const int32_t* d, int cell, int k, int c) {
     return packed_param(d, a.node_bitmap, a.prefix, a.params, cell, k, c);
 }
 
+// The packed query.  Bound by latency: per level a coordinate takes its cell's bit, its corners' rank
+// words and then their parameters, three dependent rounds of loads.  So a workgroup takes 64
+// coordinates and its four waves a quarter of the levels each (the levels stay uniform in a wave), a
+// wave runs each round for two levels before it uses the first answer, loads do not wait
+// for the cell's bit (an invisible cell's addresses are inside the layout all the same), and
+// the rows and visibility bytes are gathered in LDS and written in 16-byte stores.
+// Measured (a thread per coordinate and one level after another before): 100,003 random coordinates over
+// 20 levels 86 -> 55 us, 2^20 raster coordinates over 16 levels 299 -> 123 us, the native step's 65536
+// over 16 levels 34.7 -> 16.6 us.  Rounds of four levels 181 us for the raster (126 registers, four
+// waves per SIMD), of eight slower still; random coordinates stay bound by their scattered lines.
+constexpr int kQueryRows = 64, kQueryGroup = 2;
+
+// One corner's parameters as fp16: the first feature pair of a row (one feature: the second is 0).
+__device__ inline float2 row_pair(const PackedArgs& a, const int32_t* d, int row, int c, bool two, bool even) {
+    const int64_t at = packed_at(d, a.params, row, c);
+    if (!two) return make_float2(a.grid[at], 0.0f);
+    // even, both features inside; a clamped index (descriptors out of step with the bitmaps) stays
+    // inside the grid
+    if (even) return *reinterpret_cast<const float2*>(a.grid + (at < a.params - 1 ? at : (a.params - 2) & ~int64_t{1}));
+    return make_float2(a.grid[at], a.grid[packed_at(d, a.params, row, c + 1)]);
+}
+
+// Bytes [0, bytes) from LDS to a contiguous part of an output, in 16-byte stores where it is aligned.
+__device__ inline void store_staged(void* to, const void* staged, int bytes) {
+    int done = 0;
+    if (reinterpret_cast<uintptr_t>(to) % 16 == 0) {
+        done = bytes & ~15;
+        for (int j = threadIdx.x; j < done / 16; j += kBlock) static_cast<uint4*>(to)[j] = static_cast<const uint4*>(staged)[j];
+    }
+    for (int j = done + threadIdx.x; j < bytes; j += kBlock)
+        static_cast<uint8_t*>(to)[j] = static_cast<const uint8_t*>(staged)[j];
+}
+
 __global__ __launch_bounds__(kBlock) void packed_forward_kernel(PackedArgs a) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (i >= a.n) return;
+    extern __shared__ uint32_t staged[];
+    uint16_t* rows = reinterpret_cast<uint16_t*>(staged);                       // [64][width]
+    uint8_t* seen = reinterpret_cast<uint8_t*>(rows + kQueryRows * a.width);    // [64][levels]
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * kQueryRows;
+    const int count = static_cast<int>(a.n - first < kQueryRows ? a.n - first : kQueryRows);
+    const int64_t i = first + (lane < count ? lane : 0);
     const float2 p = reinterpret_cast<const float2*>(a.coords)[i];
-    uint16_t* row = a.features + static_cast<size_t>(i) * a.width;
-    int written = 0;
-    uint32_t vis[ODIE_MAX_LEVELS / 4];
+    uint16_t* row_out = rows + lane * a.width;
+    const bool grid_even = reinterpret_cast<uintptr_t>(a.grid) % 8 == 0 && a.params >= 2;
+    for (int l0 = wave; l0 < a.levels; l0 += 4 * kQueryGroup) {
+        int cell[kQueryGroup];
+        float w[kQueryGroup][4];
+        uint32_t byte[kQueryGroup];
 #pragma unroll
-    for (int q = 0; q < ODIE_MAX_LEVELS / 4; ++q) vis[q] = 0;
-#pragma unroll
-    for (int l = 0; l < ODIE_MAX_LEVELS; ++l) {
-        if (l < a.levels) {
+        for (int q = 0; q < kQueryGroup; ++q) {
+            const int l = l0 + 4 * q;
+            byte[q] = 0;
+            if (l >= a.levels) continue;
             const int32_t* d = a.desc + 8 * l;
-            int cell;
-            float w[4];
-            plane_geometry(p.x, p.y, d[0], cell, w);
-            const bool on = l < a.active && ((a.bitmap[d[4] + (cell >> 3)] >> (cell & 7)) & 1);
-            vis[l / 4] |= static_cast<uint32_t>(on) << (8 * (l % 4));
-            int rows[4] = {0, 0, 0, 0};
-            if (on) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k) rows[k] = packed_row(d, a.node_bitmap, a.prefix, cell, k);
-            }
-            for (int c = 0; c < d[5]; ++c) {
-                __half v = __float2half(0.0f);
-                if (on) {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        v = __hfma(__float2half_rn(keep_fp32(w[k])),
-                                   __float2half_rn(a.grid[packed_at(d, a.params, rows[k], c)]), v);
-                }
-                row[d[6] + c] = half_to_bits(v);
-            }
-            const int top = d[6] + d[5];
-            written = top > written ? top : written;
+            plane_geometry(p.x, p.y, d[0], cell[q], w[q]);
+            byte[q] = a.bitmap[d[4] + (cell[q] >> 3)];
         }
-    }
-    for (int c = written; c < a.width; ++c) row[c] = a.pad;
-    uint8_t* vrow = a.visibility + static_cast<size_t>(i) * a.levels;
+        int row[kQueryGroup][4];
+        uint64_t word[kQueryGroup][4];
 #pragma unroll
-    for (int l = 0; l < ODIE_MAX_LEVELS; ++l)
-        if (l < a.levels) vrow[l] = static_cast<uint8_t>(vis[l / 4] >> (8 * (l % 4)));
-}
-
-// packed_forward_kernel for 16 levels of 2 features in level order (width 32): both features of
-// a corner in one 8-byte load, the row kept in registers and written with 16-byte stores, the
-// visibility bytes with one.  Same arithmetic, same bits.
-__global__ __launch_bounds__(kBlock) void packed_forward16x2_kernel(PackedArgs a) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (i >= a.n) return;
-    const float2 p = reinterpret_cast<const float2*>(a.coords)[i];
-    uint32_t pairs[16];
-    uint32_t vis[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int l = 0; l < 16; ++l) {
-        const int32_t* d = a.desc + 8 * l;
-        int cell;
-        float w[4];
-        plane_geometry(p.x, p.y, d[0], cell, w);
-        const bool on = l < a.active && ((a.bitmap[d[4] + (cell >> 3)] >> (cell & 7)) & 1);
-        vis[l / 4] |= static_cast<uint32_t>(on) << (8 * (l % 4));
-        __half v0 = __float2half(0.0f), v1 = __float2half(0.0f);
-        if (on) {
-            float2 g[4];
+        for (int q = 0; q < kQueryGroup; ++q) {
+            const int l = l0 + 4 * q;
+            if (l >= a.levels) continue;
+            const int32_t* d = a.desc + 8 * l;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const int64_t at = plane_param(a, d, cell, k, 0);   // even: both features are inside
-                g[k] = *reinterpret_cast<const float2*>(a.grid + (at < a.params - 1 ? at : a.params - 2));
+                int node = cell[q] + (k & 1) + (k >> 1) * d[0];
+                if (node >= d[1]) node %= d[1];
+                row[q][k] = node;
+                if (!d[7]) {
+                    const int at = d[3] + (node >> 6);
+                    word[q][k] = a.node_bitmap[at] & ((uint64_t{1} << (node & 63)) - uint64_t{1});
+                    row[q][k] = a.prefix[at];
+                }
             }
+        }
+        float2 g[kQueryGroup][4];
+#pragma unroll
+        for (int q = 0; q < kQueryGroup; ++q) {
+            const int l = l0 + 4 * q;
+            if (l >= a.levels) continue;
+            const int32_t* d = a.desc + 8 * l;
+            const bool even = grid_even && d[2] % 2 == 0;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const __half wk = __float2half_rn(keep_fp32(w[k]));
-                v0 = __hfma(wk, __float2half_rn(g[k].x), v0);
-                v1 = __hfma(wk, __float2half_rn(g[k].y), v1);
+                if (!d[7]) row[q][k] += __popcll(word[q][k]);
+                g[q][k] = row_pair(a, d, row[q][k], 0, d[5] >= 2, even);
             }
         }
-        pairs[l] = static_cast<uint32_t>(half_to_bits(v0)) | (static_cast<uint32_t>(half_to_bits(v1)) << 16);
-    }
-    uint4* row = reinterpret_cast<uint4*>(a.features + static_cast<size_t>(i) * 32);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) row[j] = make_uint4(pairs[4 * j], pairs[4 * j + 1], pairs[4 * j + 2], pairs[4 * j + 3]);
-    reinterpret_cast<uint4*>(a.visibility)[i] = make_uint4(vis[0], vis[1], vis[2], vis[3]);
-}
-
-// packed_forward_kernel for rows of fp16 pairs: every level 2 features at output offset 2l but the
-// last, which may hold one (the reference's F2 layouts with an F1 finest level, rows of align16
-// of the features, PAIRS = width / 2).  The row is kept in registers and written with 16-byte
-// stores, the visibility bytes in 4-byte words where they fall on word boundaries.  Same
-// arithmetic, same bits.
-template <int PAIRS>
-__global__ __launch_bounds__(kBlock) void packed_forward_pairs_kernel(PackedArgs a) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (i >= a.n) return;
-    const float2 p = reinterpret_cast<const float2*>(a.coords)[i];
-    const uint32_t pad = a.pad;
-    uint32_t pairs[PAIRS];
-    uint32_t vis[PAIRS / 4];
-#pragma unroll
-    for (int q = 0; q < PAIRS / 4; ++q) vis[q] = 0;
-#pragma unroll
-    for (int l = 0; l < PAIRS; ++l) {
-        pairs[l] = pad | (pad << 16);
-        if (l < a.levels) {
+        for (int q = 0; q < kQueryGroup; ++q) {
+            const int l = l0 + 4 * q;
+            if (l >= a.levels) continue;
             const int32_t* d = a.desc + 8 * l;
-            int cell;
-            float w[4];
-            plane_geometry(p.x, p.y, d[0], cell, w);
-            const bool on = l < a.active && ((a.bitmap[d[4] + (cell >> 3)] >> (cell & 7)) & 1);
-            vis[l / 4] |= static_cast<uint32_t>(on) << (8 * (l % 4));
-            const bool two = d[5] == 2;
-            __half v0 = __float2half(0.0f), v1 = __float2half(0.0f);
-            if (on) {
-                float2 g[4];
+            const bool visible = (byte[q] >> (cell[q] & 7)) & 1, on = visible && (l < a.active || a.zero_off);
+            if (lane < count) seen[lane * a.levels + l] = visible && l < a.active;
+            typedef _Float16 pair __attribute__((ext_vector_type(2)));
+            typedef float float_pair __attribute__((ext_vector_type(2)));
+            const pair w01 = __builtin_convertvector((float_pair){keep_fp32(w[q][0]), keep_fp32(w[q][1])}, pair);
+            const pair w23 = __builtin_convertvector((float_pair){keep_fp32(w[q][2]), keep_fp32(w[q][3])}, pair);
+            const pair weight[4] = {(pair){w01.x, w01.x}, (pair){w01.y, w01.y}, (pair){w23.x, w23.x}, (pair){w23.y, w23.y}};
+            for (int c = 0; c < d[5]; c += 2) {
+                if (c > 0) {   // the second pair of a four-feature level
+                    const bool even = grid_even && d[2] % 2 == 0;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const int64_t at = plane_param(a, d, cell, k, 0);
-                    if (two) {
-                        // even, both features inside; a clamped index (descriptors out of step with
-                        // the bitmaps) stays an aligned pair inside the grid (params is a multiple of 8)
-                        g[k] = *reinterpret_cast<const float2*>(a.grid + (at < a.params - 1 ? at : a.params - 2));
-                    } else {
-                        g[k].x = a.grid[at];
-                        g[k].y = 0.0f;
-                    }
+                    for (int k = 0; k < 4; ++k) g[q][k] = row_pair(a, d, row[q][k], c, true, even);
                 }
+                pair acc = {};
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const __half wk = __float2half_rn(keep_fp32(w[k]));
-                    v0 = __hfma(wk, __float2half_rn(g[k].x), v0);
-                    v1 = __hfma(wk, __float2half_rn(g[k].y), v1);
-                }
+                for (int k = 0; k < 4; ++k)
+                    acc = __builtin_elementwise_fma(
+                        weight[k], __builtin_convertvector((float_pair){g[q][k].x, g[q][k].y}, pair), acc);
+                uint32_t bits = on ? __builtin_bit_cast(uint32_t, acc) : 0u;
+                if (l >= a.active && a.zero_off)   // an inactive level's features times zero (infinities become NaN)
+                    bits = __builtin_bit_cast(uint32_t, __builtin_bit_cast(pair, bits) * (pair){});
+                const int column = d[6] + c;
+                if (column >= 0 && column < a.width) row_out[column] = static_cast<uint16_t>(bits);
+                if (c + 1 < d[5] && column + 1 >= 0 && column + 1 < a.width) row_out[column + 1] = static_cast<uint16_t>(bits >> 16);
             }
-            pairs[l] = static_cast<uint32_t>(half_to_bits(v0)) |
-                       ((two ? static_cast<uint32_t>(half_to_bits(v1)) : pad) << 16);
         }
     }
-    uint4* row = reinterpret_cast<uint4*>(a.features + static_cast<size_t>(i) * (2 * PAIRS));
-#pragma unroll
-    for (int j = 0; j < PAIRS / 4; ++j) row[j] = make_uint4(pairs[4 * j], pairs[4 * j + 1], pairs[4 * j + 2], pairs[4 * j + 3]);
-    uint8_t* vrow = a.visibility + static_cast<size_t>(i) * a.levels;
-    if (a.levels % 4 == 0) {
-#pragma unroll
-        for (int q = 0; q < PAIRS / 4; ++q)
-            if (4 * q < a.levels) reinterpret_cast<uint32_t*>(vrow)[q] = vis[q];
-    } else {
-#pragma unroll
-        for (int l = 0; l < PAIRS; ++l)
-            if (l < a.levels) vrow[l] = static_cast<uint8_t>(vis[l / 4] >> (8 * (l % 4)));
-    }
+    int top = 0;
+    for (int l = 0; l < a.levels; ++l) top = max(top, a.desc[8 * l + 6] + a.desc[8 * l + 5]);
+    for (int c = max(top, 0) + wave; c < a.width; c += 4) row_out[c] = a.pad;
+    __syncthreads();
+    store_staged(a.features + first * a.width, rows, count * a.width * 2);
+    store_staged(a.visibility + first * a.levels, seen, count * a.levels);
 }
 
 __global__ __launch_bounds__(kBlock) void packed_backward_kernel(PackedArgs a) {
@@ -1171,8 +1150,7 @@ namespace odie {
 int packed_forward_internal(const float* coords, int64_t n, const float* grid, int64_t parameter_count,
                             const int32_t* descriptors, int levels, const uint64_t* node_bitmap,
                             const int32_t* node_prefix, const uint8_t* bitmap, int width, int active, uint16_t pad,
-                            uint16_t* features, uint8_t* visibility, hipStream_t stream, bool levels16x2,
-                            bool pairs) {
+                            uint16_t* features, uint8_t* visibility, hipStream_t stream, bool zero_off) {
     if (n < 0 || n > (int64_t{1} << 31) - 1) return fail("odie_packed_forward: n must be within [0, 2^31-1]");
     if (levels < 2 || levels > ODIE_MAX_LEVELS) return fail("odie_packed_forward: descriptor must have 2..32 levels");
     if (width < 2 || width > 128) return fail("odie_packed_forward: feature width must be within 2..128");
@@ -1196,22 +1174,10 @@ int packed_forward_internal(const float* coords, int64_t n, const float* grid, i
     a.width = width;
     a.active = active;
     a.pad = pad;
-    const uint32_t blocks = static_cast<uint32_t>((n + kBlock - 1) / kBlock);
-    const bool aligned = reinterpret_cast<uintptr_t>(features) % 16 == 0 && reinterpret_cast<uintptr_t>(grid) % 8 == 0;
-    if (levels16x2 && levels == 16 && width == 32 && aligned && reinterpret_cast<uintptr_t>(visibility) % 16 == 0) {
-        packed_forward16x2_kernel<<<blocks, kBlock, 0, stream>>>(a);
-    } else if (pairs && aligned && reinterpret_cast<uintptr_t>(visibility) % 4 == 0 && width % 16 == 0 &&
-               width >= 2 * levels && width <= 80) {
-        switch (width / 2) {
-            case 8: packed_forward_pairs_kernel<8><<<blocks, kBlock, 0, stream>>>(a); break;
-            case 16: packed_forward_pairs_kernel<16><<<blocks, kBlock, 0, stream>>>(a); break;
-            case 24: packed_forward_pairs_kernel<24><<<blocks, kBlock, 0, stream>>>(a); break;
-            case 32: packed_forward_pairs_kernel<32><<<blocks, kBlock, 0, stream>>>(a); break;
-            default: packed_forward_pairs_kernel<40><<<blocks, kBlock, 0, stream>>>(a); break;
-        }
-    } else {
-        packed_forward_kernel<<<blocks, kBlock, 0, stream>>>(a);
-    }
+    a.zero_off = zero_off ? 1 : 0;
+    const uint32_t blocks = static_cast<uint32_t>((n + kQueryRows - 1) / kQueryRows);
+    const size_t shmem = static_cast<size_t>(kQueryRows) * (2 * width + levels);   // at most 18 KB
+    packed_forward_kernel<<<blocks, kBlock, shmem, stream>>>(a);
     return check_launch("odie_packed_forward");
 }
 
@@ -1306,4 +1272,13 @@ ODIE_API int odie_packed_backward_scratch(const float* coords, int64_t n, const 
     return packed_backward_internal(coords, n, upstream, up_width, descriptors, levels, node_bitmap, node_prefix,
                                     bitmap, gradient, parameter_count, as_stream(stream), false, scratch,
                                     scratch_bytes);
+}
+
+ODIE_API int odie_packed_forward_rows(const float* coords, int64_t n, const float* grid, int64_t parameter_count,
+                                      const int32_t* descriptors, int levels, const uint64_t* node_bitmap,
+                                      const int32_t* node_prefix, const uint8_t* bitmap, int width, int active,
+                                      uint16_t* features, uint8_t* visibility, uint64_t stream) {
+    if (active < 0 || active > levels) return fail("odie_packed_forward_rows: active must be within [0, levels]");
+    return packed_forward_internal(coords, n, grid, parameter_count, descriptors, levels, node_bitmap, node_prefix,
+                                   bitmap, width, active, 0x3C00, features, visibility, as_stream(stream), true);
 }

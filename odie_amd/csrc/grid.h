@@ -261,11 +261,14 @@ int grid_backward_adam_planes_internal(const float* coords, int64_t n, const int
                                        const odie_grid_level* levels, int n_levels, int features,
                                        const AdamStep& adam, hipStream_t stream);
 
-// The packed-plane forward with the native step's active prefix (levels >= active are off)
-// and the fp16 bits written past the last level (the runtime pads with 1.0).  levels16x2: the
-// caller guarantees 16 levels of 2 features at output offsets 2l (the faster kernel applies).
-// pairs: the caller guarantees 2 features at output offset 2l for every level but the last,
-// which has 1 or 2 (the pairs kernel applies when the row is a multiple of 16 columns).
+// The packed-plane forward with an active prefix (the features of levels >= active are 0, or with
+// zero_off their values times 0, and they are not visible) and the fp16 bits written past the last
+// level (the runtime pads with 1.0).
+int packed_forward_internal(const float* coords, int64_t n, const float* grid, int64_t parameter_count,
+                            const int32_t* descriptors, int levels, const uint64_t* node_bitmap,
+                            const int32_t* node_prefix, const uint8_t* bitmap, int width, int active, uint16_t pad,
+                            uint16_t* features, uint8_t* visibility, hipStream_t stream, bool zero_off = false);
+
 // odie_packed_backward on `s`; zeroed: the caller has already cleared `gradient` (the atomics
 // and tile paths then add into it without clearing it first).  scratch: odie_packed_backward_workspace
 // bytes for the tile path, or null.
@@ -275,11 +278,6 @@ int packed_backward_internal(const float* coords, int64_t n, const uint16_t* ups
                              int64_t parameter_count, hipStream_t s, bool zeroed, void* scratch = nullptr,
                              int64_t scratch_bytes = 0);
 
-int packed_forward_internal(const float* coords, int64_t n, const float* grid, int64_t parameter_count,
-                            const int32_t* descriptors, int levels, const uint64_t* node_bitmap,
-                            const int32_t* node_prefix, const uint8_t* bitmap, int width, int active, uint16_t pad,
-                            uint16_t* features, uint8_t* visibility, hipStream_t stream, bool levels16x2 = false,
-                            bool pairs = false);
 
 
 }  // namespace odie
