@@ -448,6 +448,14 @@ int odie_gate_backward(const uint16_t* raw, const uint16_t* value, int64_t n, in
                        const int32_t* features, const uint16_t* weights, const uint8_t* visible, const float* sigmoid,
                        int coarse, int softplus, uint16_t* upstream, float* dweights, uint64_t stream);
 
+/* The evaluation's heads on feature rows [n][width] fp16 (columns past `columns` read as 1): the gate of
+ * odie_gate_forward (none with gate_weights null; levels, features, visible, coarse and softplus as
+ * there), the decoder of odie_mlp_forward, and its first three outputs as fp32 [n][3].  The same bits
+ * as those two calls. */
+int odie_heads_forward(const uint16_t* rows, int64_t n, int width, int columns, int levels, const int32_t* features,
+                       const uint16_t* gate_weights, const uint8_t* visible, int coarse, int softplus,
+                       const uint16_t* decoder_weights, float* rgb, uint64_t stream);
+
 /* ---------------------------------------------------------------------------------------
  * Stratified sampling, the device part of stratified_batches (odie/data.py:63-80): batch (a
  * square power of two, side = sqrt(batch)) slots, slot j in stratum (j % side, j / side);

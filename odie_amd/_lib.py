@@ -65,6 +65,7 @@ SIGNATURES = {
     'odie_mlp_train_planes': ([_P, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _U64], _I),
     'odie_gate_forward': ([_P, _I64, _I, _I, _P, _P, _P, _I, _I, _P, _P, _U64], _I),
     'odie_gate_backward': ([_P, _P, _I64, _I, _I, _P, _P, _P, _P, _I, _I, _P, _P, _U64], _I),
+    'odie_heads_forward': ([_P, _I64, _I, _I, _I, _P, _P, _P, _I, _I, _P, _P, _U64], _I),
     'odie_adam_step': ([_P, _P, _P, _I, _P, _P, _P, _I64, _I, _I64, C.c_float, C.c_float, C.c_float,
                         C.c_float, C.c_float, _U64], _I),
     'odie_reconstruct': ([_I64, _I64, _I, _I, _I, _I, _P, _I, _P, _I64, _P, _I, _P, _P, _P, _P, _U64], _I),

@@ -22,9 +22,9 @@ FLAGS = ['--offload-arch=' + ARCH, '-O3', '-std=c++17', '-fPIC', '-ffp-contract=
          '-I' + str(PACKAGE.parent / 'include')]
 
 
-# Per-source additions.  mlp.hip, reconstruct.hip: MFMA results in VGPRs, so the layer outputs feed
+# Per-source additions.  gate.hip, mlp.hip, reconstruct.hip: MFMA results in VGPRs, so the layer outputs feed
 # the fp16 conversions without an AGPR-to-VGPR copy per value.
-EXTRA = {source: ['-mllvm', '-amdgpu-mfma-vgpr-form'] for source in ('mlp.hip', 'reconstruct.hip')}
+EXTRA = {source: ['-mllvm', '-amdgpu-mfma-vgpr-form'] for source in ('gate.hip', 'mlp.hip', 'reconstruct.hip')}
 
 
 def hipcc():

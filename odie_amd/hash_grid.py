@@ -57,8 +57,9 @@ class HashGrid:
         """RGB fp32 [n, 3] at coordinates fp32 [n, 2] in [0, 1]^2, from the current fp32 masters
         (each call rounds them to fp16 as tiny-cuda-nn's modules do)."""
         with torch.no_grad():
-            raw = grid_forward(coordinates, self.grid.half(), self.levels, self.features_per_level)
-            return decode_rows(raw, self.gate, self.decoder)
+            raw = grid_forward(coordinates, self.grid.half(), self.levels, self.features_per_level,
+                               width=self.decoder.width)
+            return decode_rows(raw, self.gate, self.decoder, columns=self.input_width)
 
     __call__ = forward
 

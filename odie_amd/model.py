@@ -219,6 +219,12 @@ def plane_seed(seed, level):
     return (seed + 1000003 * (level + 1) + 104729 * 3) % (2 ** 31)
 
 
+def _check_query(coordinates):
+    if coordinates.dtype != torch.float32 or coordinates.ndim != 2 or coordinates.shape[1] != 2 \
+            or coordinates.requires_grad:
+        raise ValueError('Coordinates must be FP32 Nx2, without coordinate gradients')
+
+
 class PackedPlanes:
     """The packed planes of PackedXYPlanes without its heads: fp32 master `grid` in packed
     storage, the layout's addressing buffers on the device, the active prefix, and the
@@ -296,9 +302,7 @@ class PackedPlanes:
 
     def query_features(self, coordinates):
         """(features fp16 [N, input_width], visibility bool [N, L]) through PackedQuery."""
-        if coordinates.dtype != torch.float32 or coordinates.ndim != 2 or coordinates.shape[1] != 2 \
-                or coordinates.requires_grad:
-            raise ValueError('Coordinates must be FP32 Nx2, without coordinate gradients')
+        _check_query(coordinates)
         return PackedQuery.apply(coordinates.contiguous(), self.grid, self.descriptors, self.node_bitmap,
                                  self.node_prefix, self.bitmap, self.input_width)
 
@@ -328,16 +332,28 @@ def heads_match(config, gate, decoder):
     return gate_size == config['gate_parameters'] and decoder.params.numel() == config['decoder_parameters']
 
 
-def decode_rows(raw, gate, decoder, visible=None):
+def decode_rows(raw, gate, decoder, visible=None, columns=None):
     """The heads on raw features [N, sum F] fp16: columns padded with ones to the decoder's
-    width, gated per level when there is a gate, decoded; RGB fp32 [N, 3]."""
-    rows = torch.ones((raw.shape[0], decoder.width), dtype=torch.float16, device=raw.device)
-    rows[:, :raw.shape[1]] = raw
+    width, gated per level when there is a gate, decoded; RGB fp32 [N, 3].  Rows already of the
+    decoder's width are read as they are; of those, the columns past `columns` count as ones."""
+    if raw.shape[1] != decoder.width:
+        rows = torch.ones((raw.shape[0], decoder.width), dtype=torch.float16, device=raw.device)
+        rows[:, :raw.shape[1]] = raw
+        raw = rows
+    if raw.dtype != torch.float16 or not raw.is_cuda or (gate is not None and gate.width != decoder.width):
+        raise ValueError('decoder input must be CUDA fp16 [n, %d]' % decoder.width)
+    raw = raw.contiguous()
     decoder.sync_weights()
     if gate is not None:
         gate.sync_weights()
-        rows, _ = gate.forward(rows, visible=visible)
-    return decoder.forward(rows).float()[:, :3]
+    rgb = torch.empty((raw.shape[0], 3), dtype=torch.float32, device=raw.device)
+    _lib.check(_lib.library().odie_heads_forward(
+        raw.data_ptr(), raw.shape[0], decoder.width, decoder.width if columns is None else columns,
+        gate.levels if gate is not None else 0, gate._table if gate is not None else None,
+        _lib.ptr(gate.half) if gate is not None else None, _lib.ptr(visible),
+        gate.coarse if gate is not None else 0, int(gate.softplus) if gate is not None else 0,
+        decoder.half.data_ptr(), rgb.data_ptr(), _lib.stream_of(raw)))
+    return rgb
 
 
 def head_storage(grid_params, gate, decoder):
@@ -375,10 +391,18 @@ class PackedXYPlanes(PackedPlanes):
 
     def forward(self, coordinates):
         with torch.no_grad():
-            raw, visible = self.query_features(coordinates)
-            active = torch.arange(self.n_levels, device=raw.device) < self.active_prefix
-            raw = raw * active[self.feature_levels].to(raw.dtype)
-            visible = (visible & active).to(torch.uint8).contiguous()
+            _check_query(coordinates)
+            coordinates = coordinates.contiguous()
+            n, width = coordinates.shape[0], self.decoder.width
+            raw = torch.empty((n, width), dtype=torch.float16, device=coordinates.device)
+            visible = torch.empty((n, self.n_levels), dtype=torch.uint8, device=coordinates.device)
+            if self.grid.dtype != torch.float32 or self.grid.ndim != 1:
+                raise ValueError('grid must be flat CUDA FP32')
+            grid = self.grid.contiguous()
+            _lib.check(_lib.library().odie_packed_forward_rows(
+                coordinates.data_ptr(), n, grid.data_ptr(), grid.numel(), self.descriptors.data_ptr(), self.n_levels,
+                self.node_bitmap.data_ptr(), self.node_prefix.data_ptr(), self.bitmap.data_ptr(), width,
+                self.active_prefix, raw.data_ptr(), visible.data_ptr(), _lib.stream_of(coordinates)))
             return decode_rows(raw, self.gate, self.decoder, visible=visible)
 
     __call__ = forward

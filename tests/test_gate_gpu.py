@@ -12,7 +12,9 @@ import torch
 
 import oracle
 from odie_amd import synth
+from odie_amd.decoder import Decoder
 from odie_amd.gate import Gate
+from odie_amd.model import decode_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -91,3 +93,40 @@ def test_gate_backward_is_deterministic_and_empty_batch():
     gate.backward(empty, empty, torch.empty((0, 16), device='cuda'))
     torch.cuda.synchronize()
     assert not gate.grad.any()
+
+
+HEAD_ROWS = [[2] * 16, [2] * 15 + [1], [2] * 19 + [1], [2] * 20, [2] * 7 + [1], [2] * 8, [1] * 20, [4] * 12, [4] * 20,
+             [1, 4, 2, 2, 4, 1, 2, 2, 2, 4, 2, 2, 1, 2, 1, 4], [2] * 14 + [1, 2]]
+
+
+@pytest.mark.parametrize('features', HEAD_ROWS, ids=lambda f: '%dx%d' % (len(f), sum(f)))
+@pytest.mark.parametrize('n,coarse,activation,with_visible', [(1, 0, 'sigmoid', True), (33, 2, 'softplus', True),
+                                                              (4097, 0, 'sigmoid', False), (70001, 1, 'sigmoid', True)])
+def test_heads_in_one_pass_equal_the_gate_then_the_decoder(features, n, coarse, activation, with_visible):
+    """odie_heads_forward against Gate.forward and Decoder.forward, bit for bit: levels whose logits sit in
+    their columns' lanes (two features each, the last one or two) and any others, rows of every width,
+    ragged tiles, infinite and NaN features, columns past the last level."""
+    gate = Gate(seed=3, coarse=coarse, activation=activation, features=features)
+    decoder = Decoder(seed=4, width=gate.width)
+    rows = torch.from_numpy(synth.normal(5, 'heads', n * gate.width).astype(np.float16).reshape(n, gate.width)).cuda()
+    if n > 100:
+        rows[7, 1], rows[50, 0] = float('inf'), float('nan')
+    rows[:, sum(features):] = 1.0
+    visible = None
+    if with_visible:
+        visible = torch.from_numpy((synth.uniform(6, 'vis', n * len(features)) < 0.7).astype(np.uint8)
+                                   .reshape(n, len(features))).cuda()
+
+    def same(a, b):
+        assert torch.equal(a.view(torch.int32)[~torch.isnan(b)], b.view(torch.int32)[~torch.isnan(b)])
+        assert torch.equal(torch.isnan(a), torch.isnan(b))
+
+    weighted, _ = gate.forward(rows, visible=visible)
+    same(decode_rows(rows, gate, decoder, visible=visible), decoder.forward(weighted).float()[:, :3].contiguous())
+    same(decode_rows(rows, None, decoder), decoder.forward(rows).float()[:, :3].contiguous())
+    other = rows.clone()
+    other[:, sum(features):] = 0.25          # read as ones with `columns`
+    same(decode_rows(other, gate, decoder, visible=visible, columns=sum(features)),
+         decode_rows(rows, gate, decoder, visible=visible))
+    narrow = rows[:, :sum(features)]
+    same(decode_rows(narrow, gate, decoder, visible=visible), decode_rows(rows, gate, decoder, visible=visible))
