@@ -136,6 +136,10 @@ int odie_grid_backward_adam_planes(const float* coords, int64_t n, const int32_t
  * n, offsets, experts and levels, with no odie_set_tuning call in between. */
 int64_t odie_grid_handoff_bytes(int64_t n, int experts, int64_t expert_params, const odie_grid_level* levels,
                                 int n_levels, int features);
+/* The bytes of a handoff buffer that also holds the forward's own scratch: given that many,
+ * odie_grid_forward_handoff uses nothing of the library's, and may overlap other calls. */
+int64_t odie_grid_handoff_own_bytes(int64_t n, int experts, int64_t expert_params, const odie_grid_level* levels,
+                                    int n_levels, int features);
 int odie_grid_forward_handoff(const float* coords, int64_t n, const int32_t* offsets, int experts,
                               const void* params, int64_t expert_params, int param_dtype,
                               const odie_grid_level* levels, int n_levels, int features, void* out, int out_width,
@@ -170,6 +174,8 @@ int odie_grid_backward_adam_planes_handoff(const float* coords, int64_t n, const
  * most 1024 segments of 1024 counts; 0: the reduce and apply launches).  Results do
  * not depend on them beyond fp32 summation order and the owner's fixed-point scale. */
 int odie_set_tuning(const char* key, int value);
+/* How many odie_set_tuning calls have taken effect: a handoff belongs to the generation it was formed in. */
+int64_t odie_tuning_generation(void);
 
 /* ---------------------------------------------------------------------------------------
  * Packed xy planes (the on-demand representation), replacing the torch extension ops

@@ -31,8 +31,10 @@ SIGNATURES = {
                                         C.c_float, C.c_float, C.c_float, C.c_float, C.c_float, _U64], _I),
     'odie_grid_backward_planes': ([_P, _I64, _P, _I, _P, _P, _I64, _P, _I, _I, _P, _I, _U64], _I),
     'odie_set_tuning': ([C.c_char_p, _I], _I),
+    'odie_tuning_generation': ([], _I64),
     'odie_grid_forward': ([_P, _I64, _P, _I, _P, _I64, _I, _P, _I, _I, _P, _I, _U64], _I),
     'odie_grid_handoff_bytes': ([_I64, _I, _I64, _P, _I, _I], _I64),
+    'odie_grid_handoff_own_bytes': ([_I64, _I, _I64, _P, _I, _I], _I64),
     'odie_grid_forward_handoff': ([_P, _I64, _P, _I, _P, _I64, _I, _P, _I, _I, _P, _I, _P, _I64, _U64], _I),
     'odie_grid_backward_handoff': ([_P, _I64, _P, _I, _P, _I, _I, _I64, _P, _I, _I, _P, _I, _P, _I64, _U64], _I),
     'odie_grid_backward_adam_planes_handoff': ([_P, _I64, _P, _I, _P, _P, _I64, _P, _I, _I, _P, _P, _P, _P, _P,
@@ -123,9 +125,11 @@ def ptr(tensor):
 
 
 def stream_of(tensor=None):
+    """hipStream_t of the current stream on the tensor's device, as an integer (the raw handle, without
+    the Stream object torch.cuda.current_stream builds: about 2 us of a small call's host time)."""
     import torch
-    device = tensor.device if tensor is not None else None
-    return torch.cuda.current_stream(device).cuda_stream
+    index = tensor.device.index if tensor is not None else None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def set_tuning(key, value):

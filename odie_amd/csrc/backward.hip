@@ -2201,6 +2201,7 @@ int launch_owner_backward(const OwnerLaunch& in) {
         plan.ordered_at = static_cast<int64_t>(in.experts) * (kBandSlots + 1) * 4;
         plan.list_at = list_at;
         plan.sorted_at = sorted_at;
+        plan.count_bytes = static_cast<int64_t>(count_bytes);
         plan.bytes = handoff_bytes;
         return 0;
     }
@@ -2335,10 +2336,11 @@ int launch_owner_backward(const OwnerLaunch& in) {
     return check_launch("odie_grid_backward");
 }
 
-int launch_band_lists(const OwnerLaunch& in, const HandoffPlan& plan, uint8_t* handoff) {
+int launch_band_lists(const OwnerLaunch& in, const HandoffPlan& plan, uint8_t* handoff, int64_t handoff_bytes) {
     if (!plan.lists) return 0;
-    const size_t count_bytes = (static_cast<size_t>(in.experts) * plan.parts * kBandSlots * 4 + 255) / 256 * 256;
-    int32_t* counts = static_cast<int32_t*>(workspace(count_bytes, in.stream));
+    int32_t* counts = handoff_bytes >= plan.bytes + plan.count_bytes
+                          ? reinterpret_cast<int32_t*>(handoff + plan.bytes)
+                          : static_cast<int32_t*>(workspace(static_cast<size_t>(plan.count_bytes), in.stream));
     if (!counts) return -1;
     return build_band_lists(in, plan.parts, counts, reinterpret_cast<int32_t*>(handoff),
                             reinterpret_cast<int32_t*>(handoff + plan.list_at),

@@ -8,6 +8,8 @@
 // -- stay on one XCD and its L2.  The backward accumulates the coarse levels of the
 // chunk's expert in LDS (ds_add_f32) and flushes them once per chunk with global fp32
 // atomics; finer levels go straight to global_atomic_add_f32.
+#include <atomic>
+
 #include "grid.h"
 #include "adam.h"
 #include "../../include/odie_amd.h"
@@ -846,7 +848,7 @@ int grid_forward(const char* who, const float* coords, int64_t n, const int32_t*
     const hipStream_t s = as_stream(stream);
     if (plan.lists) {
         const OwnerLaunch o = planning_launch(coords, n, a.offsets, experts, expert_params, a, n_levels, features, s);
-        if (launch_band_lists(o, plan, handoff)) return -1;
+        if (launch_band_lists(o, plan, handoff, handoff_bytes)) return -1;
         a.list = reinterpret_cast<const int32_t*>(handoff + plan.list_at);
         a.sorted = reinterpret_cast<const float2*>(handoff + plan.sorted_at);
         a.ordered = reinterpret_cast<const int32_t*>(handoff + plan.ordered_at);
@@ -866,9 +868,11 @@ ODIE_API int odie_grid_forward(const float* coords, int64_t n, const int32_t* of
                         n_levels, features, out, out_width, nullptr, 0, stream);
 }
 
-ODIE_API int64_t odie_grid_handoff_bytes(int64_t n, int experts, int64_t expert_params,
-                                         const odie_grid_level* levels, int n_levels, int features) {
-    const std::string w("odie_grid_handoff_bytes");
+namespace {
+
+int64_t handoff_size(const char* who, int64_t n, int experts, int64_t expert_params, const odie_grid_level* levels,
+                     int n_levels, int features, bool own) {
+    const std::string w(who);
     if (n < 0 || n > (int64_t{1} << 31) - 1) return fail(w + ": n must be within [0, 2^31-1]");
     if (experts < 1) return fail(w + ": experts must be >= 1");
     if (!levels) return fail(w + ": levels is null");
@@ -877,13 +881,25 @@ ODIE_API int64_t odie_grid_handoff_bytes(int64_t n, int experts, int64_t expert_
         return fail(w + ": features per level must be 1, 2, 4 or 8");
     GridArgs a{};
     uint64_t entries = 0;
-    if (make_dev_levels("odie_grid_handoff_bytes", levels, n_levels, a.level, entries)) return -1;
+    if (make_dev_levels(who, levels, n_levels, a.level, entries)) return -1;
     if (expert_params < static_cast<int64_t>(entries) * features)
         return fail(w + ": expert_params is smaller than the levels' table");
     if (n == 0) return 0;
     HandoffPlan plan;
     if (handoff_plan(n, experts, expert_params, a, n_levels, features, plan)) return -1;
-    return plan.bytes;
+    return plan.bytes + (own ? plan.count_bytes : 0);
+}
+
+}  // namespace
+
+ODIE_API int64_t odie_grid_handoff_bytes(int64_t n, int experts, int64_t expert_params,
+                                         const odie_grid_level* levels, int n_levels, int features) {
+    return handoff_size("odie_grid_handoff_bytes", n, experts, expert_params, levels, n_levels, features, false);
+}
+
+ODIE_API int64_t odie_grid_handoff_own_bytes(int64_t n, int experts, int64_t expert_params,
+                                             const odie_grid_level* levels, int n_levels, int features) {
+    return handoff_size("odie_grid_handoff_own_bytes", n, experts, expert_params, levels, n_levels, features, true);
 }
 
 ODIE_API int odie_grid_forward_handoff(const float* coords, int64_t n, const int32_t* offsets, int experts,
@@ -1139,10 +1155,15 @@ ODIE_API int odie_grid_backward_planes(const float* coords, int64_t n, const int
                          as_stream(stream));
 }
 
+static std::atomic<int64_t> tuning_generation{0};
+
+ODIE_API int64_t odie_tuning_generation(void) { return tuning_generation.load(); }
+
 ODIE_API int odie_set_tuning(const char* key, int value) {
     if (!key) return fail("odie_set_tuning: key is null");
-    if (std::string(key).rfind("route_", 0) == 0) return set_route_tuning(key, value);
-    return set_grid_tuning(key, value);
+    const int status = std::string(key).rfind("route_", 0) == 0 ? set_route_tuning(key, value) : set_grid_tuning(key, value);
+    if (status == 0) tuning_generation.fetch_add(1);
+    return status;
 }
 
 namespace odie {

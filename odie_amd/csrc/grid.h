@@ -199,6 +199,7 @@ struct HandoffPlan {
     int parts;        // band counting parts per expert
     int64_t ordered_at, list_at, sorted_at;
     int64_t bytes;    // the handoff buffer's length
+    int64_t count_bytes;
 };
 
 struct OwnerLaunch {
@@ -232,7 +233,7 @@ struct OwnerLaunch {
 int launch_owner_backward(const OwnerLaunch& launch);
 // The band lists of a banded plan into `handoff` (plan.lists), for the forward to walk and the
 // backward to reuse: the owner's own band kernels on in.coords / in.offsets.
-int launch_band_lists(const OwnerLaunch& in, const HandoffPlan& plan, uint8_t* handoff);
+int launch_band_lists(const OwnerLaunch& in, const HandoffPlan& plan, uint8_t* handoff, int64_t handoff_bytes);
 
 // Owner-computes backward of packed xy planes (backward.hip): gradient [params] fp32, every
 // value written once.  upstream fp16 [n][width]; descriptors device [levels][8].

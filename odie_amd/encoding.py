@@ -105,22 +105,38 @@ def _check_handoff(handoff):
         raise ValueError('handoff must be a contiguous CUDA uint8 tensor')
 
 
+HANDOFF_BATCH = 65536
+
+
 class _GridEncode(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, coords, params, module):
+    def forward(ctx, coords, params, module, train):
         table = params if module.dtype == torch.float32 else params.to(module.dtype)
-        ctx.save_for_backward(coords)
+        # what the backward would form again in passes of its own (its band lists or slice masks)
+        # comes from the forward, which walks the lists itself; like the coordinates it is saved
+        # for this backward alone.  Small batches are bound by the host, and the saved pass is worth
+        # less than the calls for it: 4096 coordinates 118 -> 128 us a pass with, 300007 (fp32, four
+        # features) 373 -> 350, 2^22 1350 -> 1032.
+        size = 0
+        if train and coords.shape[0] >= HANDOFF_BATCH:   # with the forward's scratch: streams stay independent
+            size = max(_lib.library().odie_grid_handoff_own_bytes(coords.shape[0], 1, module.n_params, module.levels,
+                                                                  len(module.levels), module.features), 0)
+        handoff = torch.empty(size, dtype=torch.uint8, device=coords.device) if size else None
+        ctx.save_for_backward(coords, handoff)
         ctx.module = module
+        ctx.tuning = _lib.library().odie_tuning_generation() if size else 0
         return grid_forward(coords, table, module.levels, module.features, width=module.n_output_dims,
-                            expert_params=module.n_params)
+                            expert_params=module.n_params, handoff=handoff)
 
     @staticmethod
     def backward(ctx, grad_output):
-        (coords,) = ctx.saved_tensors
+        coords, handoff = ctx.saved_tensors
         module = ctx.module
+        if handoff is not None and ctx.tuning != _lib.library().odie_tuning_generation():
+            handoff = None      # formed for another plan
         gradient = grid_backward(coords, grad_output.to(module.dtype), module.levels, module.features,
-                                 expert_params=module.n_params)
-        return None, gradient, None
+                                 expert_params=module.n_params, handoff=handoff)
+        return None, gradient, None, None
 
 
 class GridEncoding(nn.Module):
@@ -142,4 +158,5 @@ class GridEncoding(nn.Module):
         self.params = nn.Parameter(torch.zeros(self.n_params, dtype=torch.float32, device=device))
 
     def forward(self, coords):
-        return _GridEncode.apply(coords.contiguous(), self.params, self)
+        return _GridEncode.apply(coords.contiguous(), self.params, self,
+                                 torch.is_grad_enabled() and self.params.requires_grad)

@@ -697,3 +697,37 @@ def test_packed_backward_scratch_is_checked_and_ragged_streams_overlap():
         d_xy.data_ptr(), n, d_up.data_ptr(), width, dev['descriptors'].data_ptr(), 9, dev['node_bitmap'].data_ptr(),
         dev['node_prefix'].data_ptr(), dev['bitmap'].data_ptr(), gradient.data_ptr(), layout['params'],
         scratch.data_ptr(), need - 1, 0) == -1
+
+
+@pytest.mark.parametrize('n,log2,levels,features,dtype', [
+    (4096, 14, 16, 2, torch.float16), (1, 14, 16, 2, torch.float16), (70001, 16, 16, 2, torch.float16),
+    (150000, 19, 16, 2, torch.float16), (150000, 19, 12, 4, torch.float32), (60001, 17, 20, 1, torch.float32)])
+def test_grid_encoding_with_its_handoff_equals_the_plain_pair(n, log2, levels, features, dtype):
+    """GridEncoding's training forward hands the backward its lists or masks: the features and the gradient
+    of odie_grid_forward and odie_grid_backward bit for bit, also on a second backward, after a tuning
+    change in between, and without gradients."""
+    from odie_amd.encoding import GridEncoding
+    module = GridEncoding(dict(n_levels=levels, n_features_per_level=features, log2_hashmap_size=log2,
+                               base_resolution=16, per_level_scale=1.38), dtype=dtype)
+    with torch.no_grad():
+        module.params.copy_(torch.from_numpy(synth.table(31, module.n_params, -1.0, 1.0, name='enc')))
+    xy = torch.from_numpy(synth.coordinates(31, n)).cuda()
+    up = torch.from_numpy(synth.upstream(31, n, module.n_output_dims)).cuda().to(dtype)
+    table = module.params.detach().to(dtype)
+    want = grid_forward(xy, table, module.levels, features)
+    gradient = grid_backward(xy, up, module.levels, features, expert_params=module.n_params)
+    out = module(xy)
+    assert torch.equal(out.detach(), want)
+    first, = torch.autograd.grad(out, module.params, up, retain_graph=True)
+    again, = torch.autograd.grad(out, module.params, up)
+    assert torch.equal(first, gradient) and torch.equal(again, gradient)
+    out = module(xy)
+    _lib.set_tuning('banded', 0)     # another plan: the handoff is not read
+    try:
+        changed, = torch.autograd.grad(out, module.params, up)
+        plain = grid_backward(xy, up, module.levels, features, expert_params=module.n_params)
+    finally:
+        _lib.set_tuning('banded', 2)
+    assert torch.equal(changed, plain)
+    with torch.no_grad():
+        assert torch.equal(module(xy), want)
