@@ -511,6 +511,70 @@ __device__ inline void accumulate_level(const float* coords, const Elem<HALF>* p
     }
 }
 
+// The coarse-group pass of one hashed level, whose adds all land: each thread takes kNeighbours
+// consecutive coordinates and adds the contributions of neighbours with the same four entries
+// together, once.  A batch in spatial order (the stratified draw lists its strata row by row) has most
+// neighbours in one cell of a coarse level: fewer lanes add, and fewer of them to one address, where
+// LDS adds serialize.  1024 experts of 2^9-entry levels, 2^24 coordinates: step 3297 -> 2993 us
+// stratified, 3100 -> 3000 us on uniform ids (64 lanes over 128 coordinates collide less too); 16 experts,
+// 2^18 stratified 484 -> 404 us.  Four neighbours measure the same, eight 3200 us; at the dense levels
+// pairs cost the uniform 64-expert step 1% and gave the stratified ones nothing.
+constexpr int kNeighbours = 2;
+
+template <int F, bool HALF, int KIND>
+__device__ inline void accumulate_neighbours(const float* coords, const Elem<HALF>* plane, const DevLevel lv, int64_t b0,
+                                             int64_t b1, uint32_t lo, uint32_t span, const float* scale,
+                                             unsigned long long* acc) {
+    const uint32_t entries = span / F;
+    const uint32_t shift = lv.offset - lo / F;
+    for (int64_t i = b0 + kNeighbours * lane_offset<KIND>(); i < b1; i += kNeighbours * kOwnerBlock) {
+        float2 xy[kNeighbours];
+        float us[kNeighbours][F];
+#pragma unroll
+        for (int b = 0; b < kNeighbours; ++b) {
+            const int64_t at = i + b < b1 ? i + b : i;
+            xy[b] = reinterpret_cast<const float2*>(coords)[at];
+            load_upstream<F, HALF>(plane, at, scale, i + b < b1, us[b]);
+        }
+        uint32_t at[4];
+        long long sum[4][F];
+#pragma unroll
+        for (int b = 0; b < kNeighbours; ++b) {
+            float w[4];
+            uint32_t idx[4];
+            corner_geometry<KIND>(xy[b].x, xy[b].y, lv, idx, w);
+            uint32_t apart = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) apart |= b ? idx[k] ^ at[k] : 0u;
+            if (b && apart) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if (at[k] + shift >= entries) continue;
+#pragma unroll
+                    for (int c = 0; c < F; ++c)
+                        atomicAdd(acc + c * entries + at[k] + shift, static_cast<unsigned long long>(sum[k][c]));
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                at[k] = idx[k];
+#pragma unroll
+                for (int c = 0; c < F; ++c) {
+                    const long long q = round_to_int(w[k] * us[b][c]);
+                    sum[k][c] = b && !apart ? sum[k][c] + q : q;
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (at[k] + shift >= entries) continue;
+#pragma unroll
+            for (int c = 0; c < F; ++c)
+                atomicAdd(acc + c * entries + at[k] + shift, static_cast<unsigned long long>(sum[k][c]));
+        }
+    }
+}
+
 // A masked slice: each wave scans its runs of 256 of the coordinates [b0, b1) through their mask
 // bytes (the next run's bytes loaded before the current run is used), queues those with a corner
 // in block `block` of the level in a ring of kRing indices in LDS (ballot positions, no barrier:
@@ -1138,7 +1202,7 @@ __global__ __launch_bounds__(kOwnerBlock) void owner_kernel(OwnerArgs a) {
         } else {
             switch (kind) {
                 case kHashed24:
-                    if (grouped) accumulate_level<F, HALF, kHashed24, kGroupBatch>(coords, plane, lv, b0, b1, lo, span, scale, acc);
+                    if (grouped) accumulate_neighbours<F, HALF, kHashed24>(coords, plane, lv, b0, b1, lo, span, scale, acc);
                     else accumulate_level<F, HALF, kHashed24>(coords, plane, lv, b0, b1, lo, span, scale, acc);
                     break;
                 case kHashedPow2: accumulate_level<F, HALF, kHashedPow2>(coords, plane, lv, b0, b1, lo, span, scale, acc); break;
