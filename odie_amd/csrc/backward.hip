@@ -270,12 +270,11 @@ __global__ __launch_bounds__(kTransposeBlock) void transpose_half2_kernel(Transp
 // Work items.  Every expert has `items` of them, in this order: the coarse-group pass (levels
 // [0, group), when group > 0) split `group_splits` ways, then for each finer level l its
 // `slices[l]` slices, each split `splits[l]` ways (item first_item[l] + slice * splits[l] + s).
-// A split takes one share of the pass's coordinates.  Unbanded, split s of a pass walks the
-// s-th index range of the expert's coordinates and writes fp32 partial slices, summed by
-// split_reduce_kernel.  Banded, the fine passes walk only the coordinates listed in the y-band
-// slots their table rows can reach (band lists below), every pass bounds its fixed-point scale
-// over all of the expert's coordinates, and splits write the raw 64-bit sums, added exactly by
-// banded_reduce_kernel: the gradient does not depend on how a pass is split.  Every column
+// A split takes one share of the pass's coordinates: the s-th index range of the expert's, or, where
+// banded, of the coordinates listed in the y-band slots that the slice's table rows can reach (band
+// lists below).  Every pass bounds its fixed-point scale over all of the expert's coordinates, and
+// splits write the raw 64-bit sums, added exactly by split_reduce_kernel: the gradient does not
+// depend on how a pass is split.  Every column
 // (level, feature) of an expert has one fixed-point scale, from its peak over the expert's
 // coordinates (column_peaks_kernel), shared by every pass and split that covers it.
 struct OwnerArgs {
@@ -284,8 +283,7 @@ struct OwnerArgs {
     const void* planes;
     const float* blockmax;      // [records][n_levels * features]: max |upstream| per 128-row record and column
     float* grad;
-    float* partial;             // unbanded splits: fp32 [max split][experts][expert_params]
-    long long* partial64;       // banded splits: int64 [max split][experts][partial_floats]
+    long long* partial64;       // splits: int64 [max split][experts][partial_floats]
     const uint32_t* peaks;      // [experts][n_levels * features]: max |upstream| of each column over the
                                 // records that meet the expert's coordinates (float bits; NaN above all)
     int64_t partial_floats;
@@ -1215,8 +1213,8 @@ __global__ __launch_bounds__(kOwnerBlock) void owner_kernel(OwnerArgs a) {
         }
     }
     __syncthreads();
-    if (splits > 1 && a.banded) {
-        // raw 64-bit sums: banded_reduce_kernel adds the splits exactly and applies the scales
+    if (splits > 1) {
+        // raw 64-bit sums: split_reduce_kernel adds the splits exactly and applies the scales
         long long* out = a.partial64 + (static_cast<int64_t>(s) * a.experts + e) * a.partial_floats + lo;
         for (uint32_t j = threadIdx.x; j < span; j += kOwnerBlock) out[j] = static_cast<long long>(acc[planar<F>(j, span)]);
         return;
@@ -1270,27 +1268,23 @@ __global__ __launch_bounds__(kOwnerBlock) void owner_kernel(OwnerArgs a) {
         }
         return;
     }
-    float* out = splits == 1 ? a.grad + static_cast<size_t>(e) * a.expert_params + lo
-                               : a.partial + static_cast<size_t>(s) * a.experts * a.expert_params +
-                                     static_cast<size_t>(e) * a.expert_params + lo;
+    float* out = a.grad + static_cast<size_t>(e) * a.expert_params + lo;
     for (uint32_t j = threadIdx.x; j < span; j += kOwnerBlock) {
         float v = unscaled(static_cast<long long>(acc[planar<F>(j, span)]), shift_of(j));
-        if (splits == 1 && a.accumulate) v += out[j];
+        if (a.accumulate) v += out[j];
         out[j] = v;
     }
 }
 
-// Banded splits: every entry of the first partial_floats values of every expert whose pass is
+// Splits: every entry of the first partial_floats values of every expert whose pass is
 // split gets the exact sum of its splits' 64-bit partials, scaled by its column's 2^-shift (the
 // same in every pass and split of the level: each bounds it over all of the expert's
 // coordinates), and is written (added with accumulate) or handed to the optimizer step, as the
 // owner does unsplit.
-__global__ __launch_bounds__(256) void banded_reduce_kernel(OwnerArgs a) {
-    const int64_t count = static_cast<int64_t>(a.experts) * a.partial_floats;
+__global__ __launch_bounds__(256) void split_reduce_kernel(OwnerArgs a) {
     const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-    for (int64_t y = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; y < count; y += stride) {
-        const int e = static_cast<int>(y / a.partial_floats);
-        const int64_t x = y % a.partial_floats;
+    for (int e = blockIdx.y; e < a.experts; e += gridDim.y)
+    for (int64_t x = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; x < a.partial_floats; x += stride) {
         const uint32_t entry = static_cast<uint32_t>(x / a.features);
         int l = 0;
         while (l + 1 < a.n_levels && a.level[l + 1].offset <= entry) ++l;
@@ -1320,24 +1314,6 @@ __global__ __launch_bounds__(256) void banded_reduce_kernel(OwnerArgs a) {
             if (a.accumulate) v += a.grad[i];
             a.grad[i] = v;
         }
-    }
-}
-
-// Sums the split partials of the first `prefix` values of every expert (prefix = expert_params:
-// all of them) and writes the gradient or applies the optimizer step.
-__global__ __launch_bounds__(256) void split_reduce_kernel(const float* partial, float* grad, int64_t total, int splits,
-                                                           int accumulate, int fused, AdamStep adam,
-                                                           int64_t expert_params, int64_t prefix) {
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-    const int64_t count = total / expert_params * prefix;
-    for (int64_t y = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; y < count; y += stride) {
-        const int64_t x = y / prefix * expert_params + y % prefix;
-        float v = accumulate ? grad[x] : 0.0f;
-        for (int s = 0; s < splits; ++s) v += partial[static_cast<size_t>(s) * total + x];
-        if (fused)
-            adam_update(adam, x, v);
-        else
-            grad[x] = v;
     }
 }
 
@@ -2179,8 +2155,12 @@ int launch_owner_backward(const OwnerLaunch& in) {
         for (int l = group; l < L; ++l)
             o.splits[l] = ways(per * band_coverage(in.levels[l], o.slice_entries[l], o.slices[l], o.row_bits[l]), 64.0);
     } else {
-        // Too few work items to fill the GPU: every pass is split over the coordinates (and the
-        // partials summed by split_reduce_kernel).  Otherwise only the coarse-group pass may be:
+        // Too few work items to fill the GPU: every pass is split over the coordinates, down to
+        // kLeastShare of an expert's a split, below which a split's own clear and 64-bit store of
+        // its slice outweigh its adds (one step, 16 experts of 2^14 coordinates, 2^9 tables: shares
+        // of 16384 / 8192 / 4096 / 2048 / 1024 403 / 289 / 241 / 217 / 216 us; 4 of 2^14, 2^10
+        // tables: 267 / 177 / 140 / 126 / 148; 9 of 7800, 2^13 tables: 162 / 161 / 162 / 160 / 201).
+        // Otherwise only the coarse-group pass may be split:
         // it walks every coordinate through `group` fully landing levels, about group + 1 times
         // the work of a fine slice (measured: ~6x with 5 levels), and when that alone exceeds one
         // CU's share of the whole pass it would set the kernel's length, so it is cut into
@@ -2188,9 +2168,10 @@ int launch_owner_backward(const OwnerLaunch& in) {
         const int64_t per_pass = static_cast<int64_t>(in.experts) * passes;
         int splits = 1;
         bool all = false;
+        constexpr int64_t kLeastShare = 2048;
         if (per_pass < 128) {
             const int64_t want = (512 + per_pass - 1) / per_pass;
-            const int64_t most = in.n / (static_cast<int64_t>(in.experts) * 16384);
+            const int64_t most = in.n / (static_cast<int64_t>(in.experts) * kLeastShare);
             splits = static_cast<int>(want < most ? want : (most > 1 ? most : 1));
             all = true;
         } else if (group > 0) {
@@ -2230,11 +2211,8 @@ int launch_owner_backward(const OwnerLaunch& in) {
     const auto align = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
     const size_t planes_bytes = in.planes ? 0 : align(static_cast<size_t>(in.n) * L * F * elem);
     const size_t max_bytes = in.planes ? 0 : align(static_cast<size_t>(records) * L * F * 4);
-    const size_t total_params = static_cast<size_t>(in.experts) * in.expert_params;
     const bool split = max_splits > 1;
-    const size_t partial_bytes = split && !banded ? align(static_cast<size_t>(max_splits) * total_params * 4) : 0;
-    const size_t partial64_bytes =
-        split && banded ? align(static_cast<size_t>(max_splits) * in.experts * split_floats * 8) : 0;
+    const size_t partial64_bytes = split ? align(static_cast<size_t>(max_splits) * in.experts * split_floats * 8) : 0;
     const size_t peak_bytes = align(static_cast<size_t>(in.experts) * L * F * 4);
     const bool lists = banded && group < L;
     const int parts = [&] {
@@ -2275,7 +2253,7 @@ int launch_owner_backward(const OwnerLaunch& in) {
     const bool given_masks = handed && !lists;
     const bool given_lists = handed && lists;
     const size_t mask_bytes = given_masks ? 0 : static_cast<size_t>(mask_stride) * mask_args.planes;
-    const size_t sizes[] = {planes_bytes, max_bytes, partial_bytes, partial64_bytes, peak_bytes,
+    const size_t sizes[] = {planes_bytes, max_bytes, partial64_bytes, peak_bytes,
                             given_lists ? 0 : count_bytes, given_lists ? 0 : start_bytes,
                             given_lists ? 0 : list_bytes, given_lists ? 0 : sorted_bytes, mask_bytes};
     constexpr int kParts = sizeof(sizes) / sizeof(sizes[0]);
@@ -2290,24 +2268,23 @@ int launch_owner_backward(const OwnerLaunch& in) {
     const bool given = in.planes != nullptr;
     o.planes = given ? in.planes : space + at[0];
     o.blockmax = given ? in.blockmax : reinterpret_cast<float*>(space + at[1]);
-    o.partial = reinterpret_cast<float*>(space + at[2]);
-    o.partial64 = reinterpret_cast<long long*>(space + at[3]);
+    o.partial64 = reinterpret_cast<long long*>(space + at[2]);
     o.partial_floats = split_floats;
-    uint32_t* peaks = reinterpret_cast<uint32_t*>(space + at[4]);
+    uint32_t* peaks = reinterpret_cast<uint32_t*>(space + at[3]);
     o.peaks = peaks;
-    const char* lists_at = given_lists ? reinterpret_cast<const char*>(in.handoff) : space + at[6];
+    const char* lists_at = given_lists ? reinterpret_cast<const char*>(in.handoff) : space + at[5];
     o.band_start = reinterpret_cast<const int32_t*>(lists_at);
-    o.band_list = reinterpret_cast<const int32_t*>(given_lists ? lists_at + list_at : space + at[7]);
-    o.band_sorted = reinterpret_cast<const float2*>(given_lists ? lists_at + sorted_at : space + at[8]);
+    o.band_list = reinterpret_cast<const int32_t*>(given_lists ? lists_at + list_at : space + at[6]);
+    o.band_sorted = reinterpret_cast<const float2*>(given_lists ? lists_at + sorted_at : space + at[7]);
     o.ordered = reinterpret_cast<const int32_t*>(lists_at + static_cast<size_t>(in.experts) * (kBandSlots + 1) * 4);
-    o.masks = !mask_args.planes ? nullptr : given_masks ? in.handoff : reinterpret_cast<const uint8_t*>(space + at[9]);
+    o.masks = !mask_args.planes ? nullptr : given_masks ? in.handoff : reinterpret_cast<const uint8_t*>(space + at[8]);
     o.mask_stride = mask_stride;
     o.grad = in.grad;
     hipStream_t s = in.stream;
 
     if (lists && !given_lists &&
-        build_band_lists(in, parts, reinterpret_cast<int32_t*>(space + at[5]), reinterpret_cast<int32_t*>(space + at[6]),
-                         reinterpret_cast<int32_t*>(space + at[7]), reinterpret_cast<float2*>(space + at[8]),
+        build_band_lists(in, parts, reinterpret_cast<int32_t*>(space + at[4]), reinterpret_cast<int32_t*>(space + at[5]),
+                         reinterpret_cast<int32_t*>(space + at[6]), reinterpret_cast<float2*>(space + at[7]),
                          const_cast<int32_t*>(o.ordered)))
         return -1;
 
@@ -2381,21 +2358,11 @@ int launch_owner_backward(const OwnerLaunch& in) {
 #undef ODIE_BOTH
 #undef ODIE_OWNER
 #undef ODIE_TRANSPOSE
-    if (split && banded) {
-        int64_t blocks = (static_cast<int64_t>(in.experts) * split_floats + 255) / 256;
+    if (split) {
+        int64_t blocks = (split_floats + 255) / 256;
         if (blocks > 16384) blocks = 16384;
-        banded_reduce_kernel<<<static_cast<uint32_t>(blocks), 256, 0, s>>>(o);
-    } else if (split) {
-        // the group pass alone split: the expert's first values; every pass split: all levels
-        const int64_t levels_end = static_cast<int64_t>(in.levels[L - 1].offset + in.levels[L - 1].size) * F;
-        const int64_t prefix = group == L || o.splits[L - 1] > 1 ? levels_end : grouped;
-        int64_t blocks = (static_cast<int64_t>(in.experts) * prefix + 255) / 256;
-        if (blocks > 16384) blocks = 16384;
-        split_reduce_kernel<<<static_cast<uint32_t>(blocks), 256, 0, s>>>(o.partial, in.grad,
-                                                                          static_cast<int64_t>(total_params),
-                                                                          static_cast<int>(max_splits),
-                                                                          in.accumulate, o.fused, o.adam,
-                                                                          in.expert_params, prefix);
+        const dim3 grid(static_cast<uint32_t>(blocks), static_cast<uint32_t>(in.experts < 65535 ? in.experts : 65535));
+        split_reduce_kernel<<<grid, 256, 0, s>>>(o);
     }
     return check_launch("odie_grid_backward");
 }

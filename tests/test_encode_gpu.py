@@ -255,6 +255,23 @@ def test_banded_splits_are_exact(log2, experts, n):
     assert torch.equal(auto, fine) and torch.equal(auto, whole)
 
 
+@pytest.mark.parametrize('log2,experts,n', [(10, 4, 4 * 4096 - 1), (10, 4, 4 * 4096), (9, 16, 200001), (14, 1, 20000),
+                                            (14, 1, 1 << 20), (13, 9, 70001)])
+def test_unbanded_splits_are_exact(log2, experts, n):
+    """Few experts without band lists: every pass splits into shares of at least 2048 coordinates of an
+    expert's (the first size is one short of two), whose 64-bit partials add exactly: the gradient equals
+    the unsplit one (band lists, one item a pass) bit for bit, added to a gradient with accumulate."""
+    levels, params, offsets, xy, up = _expert_batch(log2 + 2, log2, experts, n, outside=True)
+    start = torch.linspace(-1, 1, experts * params, device='cuda')
+    run = lambda: [grid_backward(xy, up.half(), levels, 2, offsets=offsets, experts=experts, expert_params=params),
+                   grid_backward(xy, up.half(), levels, 2, offsets=offsets, experts=experts, expert_params=params,
+                                 gradient=start.clone(), accumulate=True)]
+    split = _tuned('banded', 0, 2, run)
+    whole = _tuned('banded', 1, 2, lambda: _tuned('split_target', 1 << 30, 0, run))
+    for got, want in zip(split, whole):
+        assert torch.equal(got, want)
+
+
 def test_banded_owner_with_unordered_offsets():
     """Offsets that decrease somewhere make the expert ranges overlap: the band lists are not
     used and the fine passes walk the experts' index ranges, as the unbanded owner does."""
