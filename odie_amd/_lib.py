@@ -124,11 +124,27 @@ def ptr(tensor):
     return None if tensor is None else tensor.data_ptr()
 
 
+def optional_bytes(size, device):
+    """uint8 scratch of `size` bytes for a path that another one can stand in for: None for no bytes,
+    or when the device has no room for them."""
+    import torch
+    if not size:
+        return None
+    try:
+        return torch.empty(size, dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
 def stream_of(tensor=None):
     """hipStream_t of the current stream on the tensor's device, as an integer (the raw handle, without
     the Stream object torch.cuda.current_stream builds: about 2 us of a small call's host time)."""
     import torch
-    index = tensor.device.index if tensor is not None else None
+    index = None
+    if tensor is not None:
+        if not tensor.is_cuda:
+            raise ValueError('Expected a cuda device, but got: %s' % tensor.device)
+        index = tensor.device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 

@@ -118,13 +118,14 @@ class _GridEncode(torch.autograd.Function):
         # less than the calls for it: 4096 coordinates 118 -> 128 us a pass with, 300007 (fp32, four
         # features) 373 -> 350, 2^22 1350 -> 1032.
         size = 0
-        if train and coords.shape[0] >= HANDOFF_BATCH:   # with the forward's scratch: streams stay independent
+        if train and coords.ndim == 2 and coords.shape[0] >= HANDOFF_BATCH:
+            # with the forward's scratch: streams stay independent
             size = max(_lib.library().odie_grid_handoff_own_bytes(coords.shape[0], 1, module.n_params, module.levels,
                                                                   len(module.levels), module.features), 0)
-        handoff = torch.empty(size, dtype=torch.uint8, device=coords.device) if size else None
+        handoff = _lib.optional_bytes(size, coords.device)
         ctx.save_for_backward(coords, handoff)
         ctx.module = module
-        ctx.tuning = _lib.library().odie_tuning_generation() if size else 0
+        ctx.tuning = _lib.library().odie_tuning_generation() if handoff is not None else 0
         return grid_forward(coords, table, module.levels, module.features, width=module.n_output_dims,
                             expert_params=module.n_params, handoff=handoff)
 

@@ -182,7 +182,8 @@ def packed_backward(coordinates, upstream, descriptors, node_bitmap, node_prefix
     gradient = torch.empty(parameter_count, dtype=torch.float32, device=coordinates.device)
     lib = _lib.library()
     need = max(int(lib.odie_packed_backward_workspace(coordinates.shape[0], upstream.shape[1])), 0)
-    scratch = torch.empty(need, dtype=torch.uint8, device=coordinates.device) if need else None
+    scratch = _lib.optional_bytes(need, coordinates.device)   # without it: the pass that needs none
+    need = need if scratch is not None else 0
     _lib.check(lib.odie_packed_backward_scratch(
         coordinates.data_ptr(), coordinates.shape[0], upstream.data_ptr(), upstream.shape[1],
         descriptors.data_ptr(), descriptors.shape[0], _nonempty(node_bitmap).data_ptr(),
@@ -206,9 +207,10 @@ class PackedQuery(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, feature_gradient, visibility_gradient):
-        if feature_gradient is None:
-            return (None,) * 7
         coordinates, descriptors, node_bitmap, node_prefix, bitmap = ctx.saved_tensors
+        if feature_gradient is None:
+            zeros = torch.zeros(ctx.param_count, dtype=torch.float32, device=coordinates.device)
+            return None, zeros, None, None, None, None, None
         gradient = packed_backward(coordinates, feature_gradient.contiguous(), descriptors, node_bitmap,
                                    node_prefix, bitmap, ctx.param_count)
         return None, gradient, None, None, None, None, None
@@ -336,7 +338,7 @@ def decode_rows(raw, gate, decoder, visible=None, columns=None):
     """The heads on raw features [N, sum F] fp16: columns padded with ones to the decoder's
     width, gated per level when there is a gate, decoded; RGB fp32 [N, 3].  Rows already of the
     decoder's width are read as they are; of those, the columns past `columns` count as ones."""
-    if raw.shape[1] != decoder.width:
+    if raw.shape[1] != decoder.width or raw.dtype != torch.float16 or raw.data_ptr() % 16:
         rows = torch.ones((raw.shape[0], decoder.width), dtype=torch.float16, device=raw.device)
         rows[:, :raw.shape[1]] = raw
         raw = rows

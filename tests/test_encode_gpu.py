@@ -748,3 +748,21 @@ def test_grid_encoding_with_its_handoff_equals_the_plain_pair(n, log2, levels, f
     assert torch.equal(changed, plain)
     with torch.no_grad():
         assert torch.equal(module(xy), want)
+
+
+def test_without_memory_for_optional_scratch(monkeypatch):
+    """No room for the tiles' scratch or the handoff: the passes that need none run instead."""
+    from odie_amd.encoding import GridEncoding
+    monkeypatch.setattr(_lib, 'optional_bytes', lambda size, device: None)
+    layout, n = _packed_layout(21, **TILE_PLANES), 2000
+    xy = torch.from_numpy(synth.coordinates(21, n)).cuda()
+    up = torch.from_numpy(synth.upstream(21, n, 22)).cuda().half()
+    got = _packed_gradient(layout, xy, up, packed_owner=0).cpu().numpy()
+    want = _without_tiles(layout, xy, up).cpu().numpy()       # the same kernel: its adds' order differs
+    assert np.allclose(got, want, rtol=1e-5, atol=1e-6 * np.abs(want).max())
+    module = GridEncoding(dict(n_levels=16, n_features_per_level=2, log2_hashmap_size=16, base_resolution=16,
+                               per_level_scale=1.38))
+    xy = torch.from_numpy(synth.coordinates(32, 70001)).cuda()
+    up = torch.from_numpy(synth.upstream(32, 70001, 32)).cuda().half()
+    got, = torch.autograd.grad(module(xy), module.params, up)
+    assert torch.equal(got, grid_backward(xy, up, module.levels, 2, expert_params=module.n_params))

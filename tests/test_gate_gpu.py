@@ -130,3 +130,14 @@ def test_heads_in_one_pass_equal_the_gate_then_the_decoder(features, n, coarse, 
          decode_rows(rows, gate, decoder, visible=visible))
     narrow = rows[:, :sum(features)]
     same(decode_rows(narrow, gate, decoder, visible=visible), decode_rows(rows, gate, decoder, visible=visible))
+
+
+def test_decode_rows_takes_any_type_and_alignment():
+    """Rows of the decoder's own width in another type or off a 16-byte boundary are copied first."""
+    gate, decoder = Gate(seed=3, features=[2] * 16), Decoder(seed=4, width=32)
+    rows = torch.from_numpy(synth.normal(8, 'rows', 100 * 32).astype(np.float16).reshape(100, 32)).cuda()
+    want = decode_rows(rows, gate, decoder)
+    shifted = torch.empty(100 * 32 + 1, dtype=torch.float16, device='cuda')[1:].view(100, 32)
+    shifted.copy_(rows)
+    assert torch.equal(decode_rows(shifted, gate, decoder), want)
+    assert torch.equal(decode_rows(rows.float(), gate, decoder), want)

@@ -143,3 +143,13 @@ def test_native_optimizer_trains_a_packed_model():
     assert not torch.equal(model.decoder.params, decoder)
     assert not torch.equal(model.gate.params, gate)
     assert not torch.equal(model.forward(xy), before)
+
+
+def test_host_coordinates_are_refused():
+    """Coordinates in host memory never reach a kernel, with or without a GPU."""
+    supports, dims, caps = _inputs(9)
+    model = PackedXYPlanes(_config(**_head_sizes(dims)), supports, dims, caps, device='cpu')
+    with pytest.raises(ValueError, match='cuda'):
+        model(torch.rand(5, 2))
+    with pytest.raises(ValueError, match='cuda'):
+        model.query_features(torch.rand(5, 2))
