@@ -505,8 +505,8 @@ def reconstruction_pass(batch, fused=True):
             'batch': None if fused else batch,
             'experts': grid.experts, 'params': grid.table.numel(), 'mse': metrics['mse'],
             'top_ids_head': ids[:8].cpu().tolist(),
-            'note': 'one odie_reconstruct_scores launch (a wave per residual tile: encode + decoder + fp64 residual '
-                    'fold in registers) and odie_topk; random tables; the reference records 38 M px/s for '
+            'note': 'one odie_reconstruct_scores launch (a workgroup per residual tile: encode + decoder + fp64 '
+                    'residual fold on chip) and odie_topk; random tables; the reference records 38 M px/s for '
                     'full-image inference + residual scoring on an RTX 3060'}
 
 

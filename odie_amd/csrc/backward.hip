@@ -515,8 +515,8 @@ __device__ inline void accumulate_level(const float* coords, const Elem<HALF>* p
 // neighbours in one cell of a coarse level: fewer lanes add, and fewer of them to one address, where
 // LDS adds serialize.  1024 experts of 2^9-entry levels, 2^24 coordinates: step 3297 -> 2993 us
 // stratified, 3100 -> 3000 us on uniform ids (64 lanes over 128 coordinates collide less too); 16 experts,
-// 2^18 stratified 484 -> 404 us.  Four neighbours measure the same, eight 3200 us; at the dense levels
-// pairs cost the uniform 64-expert step 1% and gave the stratified ones nothing.
+// 2^18 stratified, in splits of 16384 coordinates, 484 -> 404 us.  Four neighbours measure the same, eight
+// 3200 us; at the dense levels pairs cost the uniform 64-expert step 1% and gave the stratified ones nothing.
 constexpr int kNeighbours = 2;
 
 template <int F, bool HALF, int KIND>
