@@ -462,6 +462,10 @@ int odie_heads_forward(const uint16_t* rows, int64_t n, int width, int columns, 
                        const uint16_t* gate_weights, const uint8_t* visible, int coarse, int softplus,
                        const uint16_t* decoder_weights, float* rgb, uint64_t stream);
 
+/* Mean of n fp32 values (16-byte aligned) in fp64, written to mean[0] in one launch and a fixed
+ * order; NaN for n = 0. */
+int odie_mean(const float* values, int64_t n, double* mean, uint64_t stream);
+
 /* ---------------------------------------------------------------------------------------
  * Stratified sampling, the device part of stratified_batches (odie/data.py:63-80): batch (a
  * square power of two, side = sqrt(batch)) slots, slot j in stratum (j % side, j / side);

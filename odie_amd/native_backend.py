@@ -220,7 +220,9 @@ class NativeOptimizer:
         else:
             self.step_raw(ids)
             self._fetch_squares(count)
-        return self.squares[:count].double().mean()
+        mean = torch.empty((), dtype=torch.float64, device=self.squares.device)
+        _lib.check(self.lib.odie_mean(self.squares.data_ptr(), count, mean.data_ptr(), _lib.stream_of(self.squares)))
+        return mean
 
     def sync_weights(self):
         self.check(self.lib.odie_sync_weights(self.handle))

@@ -507,3 +507,22 @@ def test_hash_step_matches_oracle(router, coarse, levels, features):
         assert np.array_equal(_bits(model.grid), grid0.view(np.uint32))
         assert np.array_equal(_bits(model.decoder.params), decoder0.view(np.uint32))
         opt.close()
+
+
+@pytest.mark.parametrize('n', [0, 1, 3, 4, 4095, 4097, 32767, 32768, 65536, 1000003])
+def test_mean_in_fp64(n):
+    """odie_mean: remainders of four, and both sides of a round of eight loads a thread."""
+    values = (synth.uniform(40, 'mean', n + 1) ** 2).astype(np.float32)[:n]
+    device = torch.from_numpy(values).cuda()
+    mean = torch.zeros((), dtype=torch.float64, device='cuda')
+    _lib.check(_lib.library().odie_mean(device.data_ptr(), n, mean.data_ptr(), _lib.stream_of(mean)))
+    if n == 0:
+        assert np.isnan(mean.item())
+        return
+    want = values.astype(np.float64).mean()
+    assert abs(mean.item() - want) <= 2.0 ** -53 * n * values.astype(np.float64).sum() / n   # n fp64 roundings
+    device[n // 2] = float('inf')
+    _lib.check(_lib.library().odie_mean(device.data_ptr(), n, mean.data_ptr(), _lib.stream_of(mean)))
+    assert mean.item() == float('inf')
+    misaligned = torch.zeros(9, device='cuda')[1:]
+    assert _lib.library().odie_mean(misaligned.data_ptr(), 8, mean.data_ptr(), 0) == -1
