@@ -208,9 +208,8 @@ int odie_packed_backward(const float* coords, int64_t n, const uint16_t* upstrea
 
 /* odie_packed_backward with caller-owned device scratch of odie_packed_backward_workspace(n, up_width)
  * bytes (0 for batches that take none; -1 for arguments odie_packed_backward refuses): the
- * coordinates are sorted into spatial tiles and each plane node's sum is formed in LDS, each
- * contribution the fp32 product w * u rounded to 2^-30 of its column's largest finite |u| (fp32 sums
- * where a contribution is infinite or NaN).  Calls with their own scratch may overlap.  No
+ * coordinates are sorted into spatial tiles and each plane node's sum of the fp32 products w * u is
+ * formed in LDS in fp64.  Calls with their own scratch may overlap.  No
  * counterpart in the reference. */
 int64_t odie_packed_backward_workspace(int64_t n, int up_width);
 int odie_packed_backward_scratch(const float* coords, int64_t n, const uint16_t* upstream, int up_width,

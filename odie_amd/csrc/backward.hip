@@ -1514,12 +1514,10 @@ __global__ __launch_bounds__(256) void packed_reduce_kernel(PackedOwnerArgs a) {
 //
 // Bound by: scattered straight into memory, every contribution past the coarse planes is a global
 // fp32 atomic, about 20 G/s whatever the footprint (20 levels, 100,003 coordinates: 8 M of them,
-// 410 us).  Here they are added in LDS (64-bit fixed point at 2 T/s, as in the owner pass) and a
-// node's sum is stored once:
+// 410 us).  Here they are added in LDS and a node's sum is stored once:
 //  1. packed_bin_kernel: the coordinates counted into 32 x 32 bins of the unit square per part of
-//     the batch; every upstream column's largest finite |u|; the gradient cleared;
-//  2. packed_place_kernel: the coordinates sorted by bin (their order within a bin is free: the
-//     sums are of integers);
+//     the batch; the gradient cleared;
+//  2. packed_place_kernel: the coordinates sorted by bin, in any order within a bin;
 //  3. packed_tile_kernel: a workgroup per (level, tile of 2 x 2 bins).  At a level of R >= 49 it
 //     owns the nodes of columns first_node(2 tx) .. first_node(2 tx + 2) and the same rows, which
 //     only coordinates of its own bins and of the bin row and column before them reach (two before
@@ -1531,10 +1529,11 @@ __global__ __launch_bounds__(256) void packed_reduce_kernel(PackedOwnerArgs a) {
 // Corners that wrap -- past a row's end to the next row's first node, past the last row to the
 // first -- go to memory with atomics from the coordinate's own tile, as do the sums of the nodes
 // they can reach (column 0, row 0).
-// Scale: each column's contributions times 2^S rounded to 32 bits, S from the column's largest finite
-// |u| (quantum 2^-30 of it).  A workgroup that meets a contribution the scale does not cover (an
-// infinite or NaN upstream, weights off [0, 1] from coordinates beyond 2^31 cells or NaN) starts
-// again with fp32 sums, which carry them as the atomics do.
+// Sums: the fp32 products of the atomics, added in fp64 (ds_add_f64) and rounded once, so no node's
+// sum has fewer bits than the atomics give it, however far the magnitudes in its column lie apart,
+// and infinities and NaNs arrive as they do there.  8192 random LDS slots, T adds/s: f64 1.7, u64
+// 2.9, f32 0.2; so fp64 costs little over fixed point, whose one scale per column loses small rows
+// beside large ones, and fp32 sums would set the pass's length.
 // Measured (whole backward, us, atomics -> tiles): 20 levels of 954,016 parameters 1024 coordinates
 // 108 -> 44, 131,072 491 -> 94 (334 -> 90 in spatial order), 2^20 3393 -> 469; 8 levels 44 -> 26, 198 -> 53,
 // 1395 -> 242.  Of the 100,003-coordinate backward 7 us are the binning, 8 the placing and the
@@ -1548,7 +1547,7 @@ constexpr int kFineResolution = 49;                 // two bins span (R - 1) / 1
 constexpr int kWideResolution = 97;                 // ... and so does one bin
 constexpr int kTileLdsValues = 48 * 48 * 4;         // the largest coarse level with F = 4: 72 KB
 constexpr int kBinBlock = 1024, kTileBlock = 512;
-constexpr int kMaxBinParts = 64, kMaxPeakBlocks = 128;
+constexpr int kMaxBinParts = 64;
 constexpr int kTileFlush = 3;                       // nodes a thread stores with their row lookups in flight together
 
 struct PackedTileArgs {
@@ -1564,12 +1563,9 @@ struct PackedTileArgs {
     int levels;
     int width;
     int parts;                    // parts of the batch counted apart (and placed by a block each)
-    int peak_blocks;
     int fill_blocks;              // 0: the caller has cleared the gradient
     int splits;                   // workgroups per coarse level
     uint32_t* counts;             // [parts][kTileBins]
-    uint32_t* peaks;              // [peak_blocks][width]
-    uint32_t* bounds;             // [width]
     uint32_t* starts;             // [kTileBins + 1]
     float4* sorted;               // [n]: the coordinates sorted by bin: x, y and the index's bits
 };
@@ -1599,29 +1595,6 @@ __global__ __launch_bounds__(kBinBlock) void packed_bin_kernel(PackedTileArgs a)
         return;
     }
     block -= a.parts;
-    if (block < a.peak_blocks) {
-        // thread t takes column t % width of every (kBinBlock / width)-th row, eight loads in flight
-        const int per = kBinBlock / a.width, column = threadIdx.x % a.width, first = threadIdx.x / a.width;
-        const int64_t stride = static_cast<int64_t>(a.peak_blocks) * per;
-        uint32_t mine = 0;
-        if (first < per) {
-            for (int64_t row = static_cast<int64_t>(block) * per + first; row < a.n; row += 8 * stride) {
-                uint32_t m[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int64_t at = row + j * stride < a.n ? row + j * stride : row;
-                    m[j] = a.upstream[at * a.width + column] & 0x7fffu;
-                }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) mine = max(mine, m[j] < 0x7c00u ? m[j] : 0u);
-            }
-        }
-        if (mine) atomicMax(shared + column, mine);
-        __syncthreads();
-        if (static_cast<int>(threadIdx.x) < a.width) a.peaks[block * a.width + threadIdx.x] = shared[threadIdx.x];
-        return;
-    }
-    block -= a.peak_blocks;
     for (int64_t j = static_cast<int64_t>(block) * kBinBlock + threadIdx.x; j < a.params;
          j += static_cast<int64_t>(a.fill_blocks) * kBinBlock)
         a.gradient[j] = 0.0f;
@@ -1629,21 +1602,6 @@ __global__ __launch_bounds__(kBinBlock) void packed_bin_kernel(PackedTileArgs a)
 
 __global__ __launch_bounds__(kBinBlock) void packed_place_kernel(PackedTileArgs a) {
     __shared__ uint32_t cursor[kTileBins];
-    if (static_cast<int>(blockIdx.x) == a.parts) {
-        // the blocks' peaks, eight threads a column
-        cursor[threadIdx.x] = 0;
-        __syncthreads();
-        const int column = threadIdx.x % 128, first = threadIdx.x / 128;
-        if (column < a.width) {
-            uint32_t most = 0;
-#pragma unroll 8
-            for (int b = first; b < a.peak_blocks; b += 8) most = max(most, a.peaks[b * a.width + column]);
-            atomicMax(cursor + column, most);
-        }
-        __syncthreads();
-        if (static_cast<int>(threadIdx.x) < a.width) a.bounds[threadIdx.x] = cursor[threadIdx.x];
-        return;
-    }
     // this thread's bin: how many coordinates it holds, and how many in the parts before this one
     const int part = blockIdx.x, bin = threadIdx.x;
     uint32_t total = 0, before = 0;
@@ -1692,14 +1650,12 @@ __device__ inline int first_node(int b, int r) {
 struct TileCorner {
     int ix, iy;
     float w[4];
-    bool regular;   // weights within [0, 1]
     __device__ __forceinline__ TileCorner(float2 p, int r) {
         const float px = __builtin_fmaf(static_cast<float>(r - 1), p.x, 0.5f);
         const float py = __builtin_fmaf(static_cast<float>(r - 1), p.y, 0.5f);
         ix = static_cast<int>(floorf(px));
         iy = static_cast<int>(floorf(py));
         const float fx = px - static_cast<float>(ix), fy = py - static_cast<float>(iy);
-        regular = fx >= 0.0f && fx <= 1.0f && fy >= 0.0f && fy <= 1.0f;
         ix = ix < 0 ? 0 : (ix > r - 1 ? r - 1 : ix);
         iy = iy < 0 ? 0 : (iy > r - 1 ? r - 1 : iy);
         w[0] = (1.0f - fx) * (1.0f - fy);
@@ -1722,111 +1678,76 @@ template <int F> struct TileLevel {
     int r, points, column;
     int64_t cells;          // byte offset of the level's cell bits
     int used;               // features with an upstream column
-    int32_t shift[F];
-    float scale[F], peak[F];
 
     __device__ __forceinline__ TileLevel(const PackedTileArgs& args, const int32_t* desc)
         : a(args), d(desc), r(desc[0]), points(desc[1]), column(desc[6]), cells(desc[4]) {
         used = 0;
 #pragma unroll
-        for (int c = 0; c < F; ++c) {
-            const bool real = column + c < a.width;
-            used += real;
-            peak[c] = real ? __half2float(bits_to_half(static_cast<uint16_t>(a.bounds[column + c]))) : 0.0f;
-            shift[c] = column_shift(__float_as_uint(peak[c]), a.n);
-            scale[c] = shift_scale(shift[c]);
-        }
+        for (int c = 0; c < F; ++c) used += column + c < a.width;
     }
     __device__ __forceinline__ bool visible(int cell) const { return (a.bitmap[cells + (cell >> 3)] >> (cell & 7)) & 1; }
-    // The upstream values of row i; false when one is not within its column's finite peak.
-    __device__ __forceinline__ bool load(int64_t i, float u[F]) const {
+    // The upstream values of row i.
+    __device__ __forceinline__ void load(int64_t i, float u[F]) const {
         const uint16_t* row = a.upstream + i * a.width + column;
-        bool regular = true;
 #pragma unroll
-        for (int c = 0; c < F; ++c) {
-            u[c] = c < used ? __half2float(bits_to_half(row[c])) : 0.0f;
-            regular = regular && fabsf(u[c]) <= peak[c];
-        }
-        return regular;
+        for (int c = 0; c < F; ++c) u[c] = c < used ? __half2float(bits_to_half(row[c])) : 0.0f;
     }
     // Adds w * u of one corner to the F accumulators from slot `at`.
-    __device__ __forceinline__ void add(unsigned long long* acc, bool exact, int at, float w, const float u[F]) const {
+    __device__ __forceinline__ void add(double* acc, int at, float w, const float u[F]) const {
 #pragma unroll
-        for (int c = 0; c < F; ++c) {
-            if (u[c] == 0.0f) continue;
-            if (exact) {
-                const int32_t q = round_to_int(w * u[c] * scale[c]);
-                atomicAdd(acc + at * F + c, static_cast<unsigned long long>(static_cast<long long>(q)));
-            } else {
-                atomicAdd(reinterpret_cast<float*>(acc) + at * F + c, w * u[c]);
-            }
-        }
-    }
-    __device__ __forceinline__ float value(const unsigned long long* acc, bool exact, int slot, int c) const {
-        return exact ? unscaled(static_cast<long long>(acc[slot]), shift[c]) : reinterpret_cast<const float*>(acc)[slot];
+        for (int c = 0; c < F; ++c)
+            if (u[c] != 0.0f) atomicAdd(acc + at * F + c, static_cast<double>(w * u[c]));
     }
     __device__ __forceinline__ float* parameter(int row, int c) const { return a.gradient + packed_at(d, a.params, row, c); }
 };
 
 // A part of the batch at a coarse level: every node in LDS, the sums added to the gradient.
 template <int F>
-__device__ __forceinline__ void coarse_level(const TileLevel<F>& level, int split, unsigned long long* acc, int& irregular) {
+__device__ __forceinline__ void coarse_level(const TileLevel<F>& level, int split, double* acc) {
     const PackedTileArgs& a = level.a;
     const int64_t share = (a.n + a.splits - 1) / a.splits;
     const int64_t b0 = share * split, b1 = b0 + share < a.n ? b0 + share : a.n;
     if (b0 >= b1) return;
     const int slots = level.points * F;
-    for (int attempt = 0; attempt < 2; ++attempt) {
-        const bool exact = attempt == 0;
-        for (int j = threadIdx.x; j < slots; j += kTileBlock) acc[j] = 0;
-        if (threadIdx.x == 0) irregular = 0;
-        __syncthreads();
-        // a wave's lanes take coordinates `rows` apart: a batch in spatial order would otherwise put them
-        // on one node, and LDS adds to one address serialize
-        const int rows = static_cast<int>((b1 - b0 + 63) / 64);
-        for (int k = threadIdx.x / 64; k < rows; k += kTileBlock / 64) {
-            const int64_t i = b0 + static_cast<int64_t>(threadIdx.x % 64) * rows + k;
-            if (i >= b1) continue;
-            const TileCorner at(reinterpret_cast<const float2*>(a.coords)[i], level.r);
-            const int cell = at.ix + at.iy * level.r;
-            if (!level.visible(cell)) continue;
-            float u[F];
-            const bool regular = level.load(i, u) && at.regular;
-            if (exact && !regular) {
-                irregular = 1;
-                continue;
-            }
+    for (int j = threadIdx.x; j < slots; j += kTileBlock) acc[j] = 0.0;
+    __syncthreads();
+    // a wave's lanes take coordinates `rows` apart: a batch in spatial order would otherwise put them
+    // on one node, and LDS adds to one address serialize
+    const int rows = static_cast<int>((b1 - b0 + 63) / 64);
+    for (int k = threadIdx.x / 64; k < rows; k += kTileBlock / 64) {
+        const int64_t i = b0 + static_cast<int64_t>(threadIdx.x % 64) * rows + k;
+        if (i >= b1) continue;
+        const TileCorner at(reinterpret_cast<const float2*>(a.coords)[i], level.r);
+        const int cell = at.ix + at.iy * level.r;
+        if (!level.visible(cell)) continue;
+        float u[F];
+        level.load(i, u);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int node = cell + (k & 1) + (k >> 1) * level.r;
-                level.add(acc, exact, node < level.points ? node : node - level.points, at.w[k], u);
-            }
+        for (int k = 0; k < 4; ++k) {
+            const int node = cell + (k & 1) + (k >> 1) * level.r;
+            level.add(acc, node < level.points ? node : node - level.points, at.w[k], u);
         }
-        __syncthreads();
-        if (!exact || !irregular) {
-            for (int node = threadIdx.x; node < level.points; node += kTileBlock) {
-                float v[F];
-                bool any = false;
+    }
+    __syncthreads();
+    for (int node = threadIdx.x; node < level.points; node += kTileBlock) {
+        float v[F];
+        bool any = false;
 #pragma unroll
-                for (int c = 0; c < F; ++c) {
-                    v[c] = level.value(acc, exact, node * F + c, c);
-                    any = any || v[c] != 0.0f;
-                }
-                if (!any) continue;
-                const int row = node_row(a, level.d, node);
-#pragma unroll
-                for (int c = 0; c < F; ++c)
-                    if (v[c] != 0.0f) atomicAdd(level.parameter(row, c), v[c]);
-            }
-            return;
+        for (int c = 0; c < F; ++c) {
+            v[c] = static_cast<float>(acc[node * F + c]);
+            any = any || v[c] != 0.0f;
         }
-        __syncthreads();
+        if (!any) continue;
+        const int row = node_row(a, level.d, node);
+#pragma unroll
+        for (int c = 0; c < F; ++c)
+            if (v[c] != 0.0f) atomicAdd(level.parameter(row, c), v[c]);
     }
 }
 
 // The nodes [x0, x1) x [y0, y1) of a tile at a fine level, in pieces that fit LDS.
 template <int F>
-__device__ __forceinline__ void fine_tile(const TileLevel<F>& level, int tx, int ty, unsigned long long* acc, int& irregular) {
+__device__ __forceinline__ void fine_tile(const TileLevel<F>& level, int tx, int ty, double* acc) {
     const PackedTileArgs& a = level.a;
     const int r = level.r;
     const int x0 = first_node(2 * tx, r), x1 = first_node(2 * tx + 2, r);
@@ -1851,114 +1772,102 @@ __device__ __forceinline__ void fine_tile(const TileLevel<F>& level, int tx, int
     for (int py = y0; py < y1; py += piece_y)
         for (int px = x0; px < x1; px += piece_x) {
             const int nx = min(piece_x, x1 - px), ny = min(piece_y, y1 - py);
-            for (int attempt = 0; attempt < 2; ++attempt) {
-                const bool exact = attempt == 0;
-                __syncthreads();
-                for (int j = threadIdx.x; j < nx * ny * F; j += kTileBlock) acc[j] = 0;
-                if (threadIdx.x == 0) irregular = 0;
-                __syncthreads();
-                for (int64_t j = threadIdx.x; j < total; j += kTileBlock) {
-                    int64_t pos = from[0] + j;
-                    pos = j >= upto[0] ? from[1] + j - upto[0] : pos;
-                    pos = j >= upto[1] ? from[2] + j - upto[1] : pos;
-                    pos = j >= upto[2] ? from[3] + j - upto[2] : pos;
-                    const float4 entry = a.sorted[pos];
-                    const float2 p = make_float2(entry.x, entry.y);
-                    const TileCorner at(p, r);
-                    const int lx = at.ix - px, ly = at.iy - py;   // inside: corners lx, lx + 1 in [0, nx)
-                    const bool inside = lx >= -1 && lx < nx && ly >= -1 && ly < ny;
-                    const bool wraps = exact && first && (at.ix == r - 1 || at.iy == r - 1) &&
-                                       (bin_of(p.x) >> 1) == tx && (bin_of(p.y) >> 1) == ty;
-                    if (!inside && !wraps) continue;
-                    const int cell = at.ix + at.iy * r;
-                    float u[F];   // loaded beside the cell's bit, not after it
-                    const bool seen = level.visible(cell);
-                    const bool regular = level.load(__float_as_uint(entry.z), u) && at.regular;
-                    if (!seen) continue;
-                    if (inside) {
-                        if (exact && !regular) {
-                            irregular = 1;
+            __syncthreads();
+            for (int j = threadIdx.x; j < nx * ny * F; j += kTileBlock) acc[j] = 0.0;
+            __syncthreads();
+            for (int64_t j = threadIdx.x; j < total; j += kTileBlock) {
+                int64_t pos = from[0] + j;
+                pos = j >= upto[0] ? from[1] + j - upto[0] : pos;
+                pos = j >= upto[1] ? from[2] + j - upto[1] : pos;
+                pos = j >= upto[2] ? from[3] + j - upto[2] : pos;
+                const float4 entry = a.sorted[pos];
+                const float2 p = make_float2(entry.x, entry.y);
+                const TileCorner at(p, r);
+                const int lx = at.ix - px, ly = at.iy - py;   // inside: corners lx, lx + 1 in [0, nx)
+                const bool inside = lx >= -1 && lx < nx && ly >= -1 && ly < ny;
+                const bool wraps = first && (at.ix == r - 1 || at.iy == r - 1) &&
+                                   (bin_of(p.x) >> 1) == tx && (bin_of(p.y) >> 1) == ty;
+                if (!inside && !wraps) continue;
+                const int cell = at.ix + at.iy * r;
+                float u[F];   // loaded beside the cell's bit, not after it
+                const bool seen = level.visible(cell);
+                level.load(__float_as_uint(entry.z), u);
+                if (!seen) continue;
+                if (inside) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int cx = lx + (k & 1), cy = ly + (k >> 1);
+                        const bool here = cx >= 0 && cx < nx && cy >= 0 && cy < ny;
+                        if (here) level.add(acc, cy * nx + cx, at.w[k], u);
+                    }
+                }
+                if (wraps) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if (at.ix + (k & 1) < r && at.iy + (k >> 1) < r) continue;
+                        const int node = (cell + (k & 1) + (k >> 1) * r) % level.points;
+                        const int row = node_row(a, level.d, node);
+#pragma unroll
+                        for (int c = 0; c < F; ++c)
+                            if (u[c] != 0.0f) atomicAdd(level.parameter(row, c), at.w[k] * u[c]);
+                    }
+                }
+            }
+            __syncthreads();
+            for (int j0 = threadIdx.x; j0 < nx * ny; j0 += kTileFlush * kTileBlock) {
+                float v[kTileFlush][F];
+                int row[kTileFlush], node[kTileFlush];
+#pragma unroll
+                for (int q = 0; q < kTileFlush; ++q) {
+                    const int j = j0 + q * kTileBlock;
+                    bool any = false;
+#pragma unroll
+                    for (int c = 0; c < F; ++c) {
+                        v[q][c] = j < nx * ny ? static_cast<float>(acc[j * F + c]) : 0.0f;
+                        any = any || v[q][c] != 0.0f;
+                    }
+                    node[q] = any ? px + j % nx + (py + j / nx) * r : -1;
+                    row[q] = any ? node_row(a, level.d, node[q]) : 0;
+                }
+#pragma unroll
+                for (int q = 0; q < kTileFlush; ++q) {
+                    if (node[q] < 0) continue;
+                    const bool shared_node = node[q] < r || node[q] % r == 0;
+#pragma unroll
+                    for (int c = 0; c < F; ++c) {
+                        if (shared_node) {
+                            if (v[q][c] != 0.0f) atomicAdd(level.parameter(row[q], c), v[q][c]);
                         } else {
-#pragma unroll
-                            for (int k = 0; k < 4; ++k) {
-                                const int cx = lx + (k & 1), cy = ly + (k >> 1);
-                                const bool here = cx >= 0 && cx < nx && cy >= 0 && cy < ny;
-                                if (here) level.add(acc, exact, cy * nx + cx, at.w[k], u);
-                            }
-                        }
-                    }
-                    if (wraps) {
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) {
-                            if (at.ix + (k & 1) < r && at.iy + (k >> 1) < r) continue;
-                            const int node = (cell + (k & 1) + (k >> 1) * r) % level.points;
-                            const int row = node_row(a, level.d, node);
-#pragma unroll
-                            for (int c = 0; c < F; ++c)
-                                if (u[c] != 0.0f) atomicAdd(level.parameter(row, c), at.w[k] * u[c]);
+                            *level.parameter(row[q], c) = v[q][c];
                         }
                     }
                 }
-                __syncthreads();
-                if (exact && irregular) continue;
-                for (int j0 = threadIdx.x; j0 < nx * ny; j0 += kTileFlush * kTileBlock) {
-                    float v[kTileFlush][F];
-                    int row[kTileFlush], node[kTileFlush];
-#pragma unroll
-                    for (int q = 0; q < kTileFlush; ++q) {
-                        const int j = j0 + q * kTileBlock;
-                        bool any = false;
-#pragma unroll
-                        for (int c = 0; c < F; ++c) {
-                            v[q][c] = j < nx * ny ? level.value(acc, exact, j * F + c, c) : 0.0f;
-                            any = any || v[q][c] != 0.0f;
-                        }
-                        node[q] = any ? px + j % nx + (py + j / nx) * r : -1;
-                        row[q] = any ? node_row(a, level.d, node[q]) : 0;
-                    }
-#pragma unroll
-                    for (int q = 0; q < kTileFlush; ++q) {
-                        if (node[q] < 0) continue;
-                        const bool shared_node = node[q] < r || node[q] % r == 0;
-#pragma unroll
-                        for (int c = 0; c < F; ++c) {
-                            if (shared_node) {
-                                if (v[q][c] != 0.0f) atomicAdd(level.parameter(row[q], c), v[q][c]);
-                            } else {
-                                *level.parameter(row[q], c) = v[q][c];
-                            }
-                        }
-                    }
-                }
-                break;
             }
             first = false;
         }
 }
 
 template <int F>
-__device__ __forceinline__ void tile_level(const PackedTileArgs& a, const int32_t* d, int slot, unsigned long long* acc,
-                                  int& irregular) {
+__device__ __forceinline__ void tile_level(const PackedTileArgs& a, const int32_t* d, int slot, double* acc) {
     const TileLevel<F> level(a, d);
     if (level.used == 0) return;
     if (level.r < kFineResolution) {
-        if (slot < a.splits) coarse_level(level, slot, acc, irregular);
+        if (slot < a.splits) coarse_level(level, slot, acc);
         return;
     }
     // consecutive tiles on one XCD (a block's XCD is its index mod 8), so that they share its L2
     const int tile = (slot % kXcds) * (kTiles / kXcds) + slot / kXcds;
-    fine_tile(level, tile % kTileSide, tile / kTileSide, acc, irregular);
+    fine_tile(level, tile % kTileSide, tile / kTileSide, acc);
 }
 
 __global__ __launch_bounds__(kTileBlock) void packed_tile_kernel(PackedTileArgs a) {
-    extern __shared__ unsigned long long acc[];
-    __shared__ int irregular;
+    extern __shared__ double sums[];
     const int slot = blockIdx.x % kTiles;
     const int32_t* d = a.desc + 8 * (blockIdx.x / kTiles);
     switch (d[5]) {
-        case 1: tile_level<1>(a, d, slot, acc, irregular); break;
-        case 2: tile_level<2>(a, d, slot, acc, irregular); break;
-        case 4: tile_level<4>(a, d, slot, acc, irregular); break;
+        case 1: tile_level<1>(a, d, slot, sums); break;
+        case 2: tile_level<2>(a, d, slot, sums); break;
+        case 4: tile_level<4>(a, d, slot, sums); break;
         default: break;
     }
 }
@@ -2381,16 +2290,13 @@ int launch_band_lists(const OwnerLaunch& in, const HandoffPlan& plan, uint8_t* h
 
 namespace {
 
-struct TileLayout { size_t peaks, bounds, starts, sorted, total; int parts, peak_blocks; };
+struct TileLayout { size_t starts, sorted, total; int parts; };
 
-TileLayout tile_layout(int64_t n, int width) {
+TileLayout tile_layout(int64_t n) {
     const auto align = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
     TileLayout l{};
     l.parts = static_cast<int>(std::min<int64_t>(std::max<int64_t>(n / 2048, 1), kMaxBinParts));
-    l.peak_blocks = static_cast<int>(std::min<int64_t>(std::max<int64_t>(n / 512, 1), kMaxPeakBlocks));
-    l.peaks = align(sizeof(uint32_t) * l.parts * kTileBins);
-    l.bounds = l.peaks + align(sizeof(uint32_t) * l.peak_blocks * width);
-    l.starts = l.bounds + align(sizeof(uint32_t) * width);
+    l.starts = align(sizeof(uint32_t) * l.parts * kTileBins);
     l.sorted = l.starts + align(sizeof(uint32_t) * (kTileBins + 1));
     l.total = l.sorted + align(sizeof(float4) * n);
     return l;
@@ -2398,12 +2304,12 @@ TileLayout tile_layout(int64_t n, int width) {
 
 }  // namespace
 
-int64_t packed_tile_workspace(int64_t n, int width) { return static_cast<int64_t>(tile_layout(n, width).total); }
+int64_t packed_tile_workspace(int64_t n) { return static_cast<int64_t>(tile_layout(n).total); }
 
 int launch_packed_tiles(const float* coords, int64_t n, const uint16_t* upstream, int width, const int32_t* desc,
                         int levels, const uint64_t* node_bitmap, const int32_t* node_prefix, const uint8_t* bitmap,
                         float* gradient, int64_t params, bool zeroed, void* workspace, hipStream_t stream) {
-    const TileLayout l = tile_layout(n, width);
+    const TileLayout l = tile_layout(n);
     char* space = static_cast<char*>(workspace);
     PackedTileArgs a{};
     a.coords = coords;
@@ -2418,18 +2324,15 @@ int launch_packed_tiles(const float* coords, int64_t n, const uint16_t* upstream
     a.levels = levels;
     a.width = width;
     a.parts = l.parts;
-    a.peak_blocks = l.peak_blocks;
     a.fill_blocks = zeroed ? 0 : static_cast<int>(std::min<int64_t>((params + kBinBlock - 1) / kBinBlock, kCus));
     a.splits = static_cast<int>(std::min<int64_t>(std::max<int64_t>(n / 2048, 1), 32));
     a.counts = reinterpret_cast<uint32_t*>(space);
-    a.peaks = reinterpret_cast<uint32_t*>(space + l.peaks);
-    a.bounds = reinterpret_cast<uint32_t*>(space + l.bounds);
     a.starts = reinterpret_cast<uint32_t*>(space + l.starts);
     a.sorted = reinterpret_cast<float4*>(space + l.sorted);
-    constexpr size_t shmem = sizeof(unsigned long long) * kTileLdsValues;
+    constexpr size_t shmem = sizeof(double) * kTileLdsValues;
     if (allow_lds(packed_tile_kernel, shmem)) return -1;
-    packed_bin_kernel<<<static_cast<uint32_t>(a.parts + a.peak_blocks + a.fill_blocks), kBinBlock, 0, stream>>>(a);
-    packed_place_kernel<<<static_cast<uint32_t>(a.parts + 1), kBinBlock, 0, stream>>>(a);
+    packed_bin_kernel<<<static_cast<uint32_t>(a.parts + a.fill_blocks), kBinBlock, 0, stream>>>(a);
+    packed_place_kernel<<<static_cast<uint32_t>(a.parts), kBinBlock, 0, stream>>>(a);
     packed_tile_kernel<<<static_cast<uint32_t>(levels * kTiles), kTileBlock, shmem, stream>>>(a);
     return check_launch("odie_packed_backward");
 }

@@ -1239,7 +1239,7 @@ int packed_backward_internal(const float* coords, int64_t n, const uint16_t* ups
         return launch_packed_owner(coords, n, upstream, up_width, descriptors, levels, node_bitmap, node_prefix, bitmap,
                                    gradient, parameter_count, t.owner_lds_bytes, t.packed_splits, s);
     if (scratch && t.packed_tiles && n >= kTiledBatch) {
-        if (scratch_bytes < packed_tile_workspace(n, up_width) || reinterpret_cast<uintptr_t>(scratch) % 16)
+        if (scratch_bytes < packed_tile_workspace(n) || reinterpret_cast<uintptr_t>(scratch) % 16)
             return fail("odie_packed_backward: scratch must be aligned and hold odie_packed_backward_workspace bytes");
         return launch_packed_tiles(coords, n, upstream, up_width, descriptors, levels, node_bitmap, node_prefix,
                                    bitmap, gradient, parameter_count, zeroed, scratch, s);
@@ -1282,7 +1282,7 @@ ODIE_API int odie_packed_backward(const float* coords, int64_t n, const uint16_t
 
 ODIE_API int64_t odie_packed_backward_workspace(int64_t n, int up_width) {
     if (n < 0 || n > (int64_t{1} << 31) - 1 || up_width < 2 || up_width > 128) return -1;
-    return n < kTiledBatch ? 0 : packed_tile_workspace(n, up_width);
+    return n < kTiledBatch ? 0 : packed_tile_workspace(n);
 }
 
 ODIE_API int odie_packed_backward_scratch(const float* coords, int64_t n, const uint16_t* upstream, int up_width,

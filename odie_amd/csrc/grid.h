@@ -242,8 +242,8 @@ int launch_packed_owner(const float* coords, int64_t n, const uint16_t* upstream
                         float* gradient, int64_t params, int64_t lds_bytes, int64_t splits, hipStream_t stream);
 
 // The same gradient by spatial tiles (backward.hip), with scratch of packed_tile_workspace bytes;
-// zeroed: the caller has cleared the gradient.  width <= 128.
-int64_t packed_tile_workspace(int64_t n, int width);
+// zeroed: the caller has cleared the gradient.
+int64_t packed_tile_workspace(int64_t n);
 int launch_packed_tiles(const float* coords, int64_t n, const uint16_t* upstream, int width, const int32_t* desc,
                         int levels, const uint64_t* node_bitmap, const int32_t* node_prefix, const uint8_t* bitmap,
                         float* gradient, int64_t params, bool zeroed, void* workspace, hipStream_t stream);

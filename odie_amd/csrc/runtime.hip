@@ -442,7 +442,7 @@ Runtime::Runtime(const Json& j)
     vis.allocate(static_cast<size_t>(levels) * kBatch);
     flag.allocate(1);
     grid_grad.allocate(total);
-    if (!hash) packed_scratch.allocate(packed_tile_workspace(kBatch, row));
+    if (!hash) packed_scratch.allocate(packed_tile_workspace(kBatch));
     grid_grad.zero(stream);
     grid_adam.allocate(total, stream);
     decoder.reset(new Head(device_pointer<float>(j, "decoder"), decoder_params(row), stream));

@@ -658,6 +658,28 @@ def test_packed_tiles_column_scales_and_zero_upstream():
     assert not bool(zero.any())
 
 
+@pytest.mark.parametrize('case', ['outlier', 'alternate'])
+def test_packed_tiles_rows_of_one_column_far_apart(case):
+    """Rows of one column 2^20 and more apart: every node keeps the bits that fp32 sums of its own
+    contributions have, whatever the largest row of its column is."""
+    layout = _packed_layout(25, **TILE_PLANES)
+    n, width = 20000, 22
+    xy = synth.coordinates(25, n)
+    up = synth.upstream(25, n, width).astype(np.float32)
+    up *= (1e-2 if case == 'outlier' else np.where(np.arange(n) % 2 == 0, 2.0 ** 10, 2.0 ** -10)[:, None]) / np.abs(up).max()
+    if case == 'outlier':
+        up[7] = 6e4
+    up = up.astype(np.float16)
+    host = {k: layout[k].numpy() for k in ('descriptors', 'node_bitmap', 'node_prefix', 'bitmap')}
+    expected, magnitude, counts = oracle.packed_backward(xy, up, host, layout['params'], counts=True)
+    got = _packed_gradient(layout, torch.from_numpy(xy).cuda(), torch.from_numpy(up).cuda(), packed_owner=0)
+    # an fp32 rounding for each contribution that goes to memory by itself, or for each of a node's
+    # at most 32 partial sums, and one for the sum
+    bound = (counts + 33) * 2.0 ** -24 * magnitude
+    error = np.abs(got.cpu().numpy().astype(np.float64) - expected)
+    assert (error <= bound).all(), (error / np.maximum(bound, 1e-300)).max()
+
+
 @pytest.mark.parametrize('case', ['inf', 'nan', 'nan_xy', 'far_xy', 'all_inf'])
 def test_packed_tiles_carry_infinities_and_nans_as_the_atomics_do(case):
     layout = _packed_layout(23, **TILE_PLANES)
