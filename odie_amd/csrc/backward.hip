@@ -1525,7 +1525,7 @@ __global__ __launch_bounds__(256) void packed_reduce_kernel(PackedOwnerArgs a) {
 //     their corners one further).  It adds their corners in LDS and stores the nodes that are not
 //     zero.  Coarser
 //     levels (at most 48^2 nodes) are summed by up to 32 workgroups over parts of the batch and added
-//     with atomics.
+//     with atomics.  Planes too fine for it (tiled_level) take the atomics, in the sorted order.
 // Corners that wrap -- past a row's end to the next row's first node, past the last row to the
 // first -- go to memory with atomics from the coordinate's own tile, as do the sums of the nodes
 // they can reach (column 0, row 0).
@@ -1534,12 +1534,10 @@ __global__ __launch_bounds__(256) void packed_reduce_kernel(PackedOwnerArgs a) {
 // and infinities and NaNs arrive as they do there.  8192 random LDS slots, T adds/s: f64 1.7, u64
 // 2.9, f32 0.2; so fp64 costs little over fixed point, whose one scale per column loses small rows
 // beside large ones, and fp32 sums would set the pass's length.
-// Measured (whole backward, us, atomics -> tiles): 20 levels of 954,016 parameters 1024 coordinates
-// 108 -> 44, 131,072 491 -> 94 (334 -> 90 in spatial order), 2^20 3393 -> 469; 8 levels 44 -> 26, 198 -> 53,
-// 1395 -> 242.  Of the 100,003-coordinate backward 7 us are the binning, 8 the placing and the
-// clearing's share, 75 the tiles: chains of dependent loads (list entry, cell bit and upstream; then the
-// node's prefix and word) in two workgroups of eight waves per CU, whose LDS a 1020-cell level fills.
-// Workgroups of 1024 threads: 20 us slower (one per CU at these registers).
+// Measured: the whole backward at kTiledBatch (encode.hip).  The tile kernel waits on chains of dependent
+// loads (list entry, cell bit and upstream; then the node's prefix and word) in two workgroups of eight
+// waves per CU, whose LDS a 1020-cell level fills.  Workgroups of 1024 threads: 20 us slower for 100,003
+// coordinates over 20 levels (one per CU at these registers).
 // ---------------------------------------------------------------------------------------
 constexpr int kBinSide = 32, kTileBins = kBinSide * kBinSide;
 constexpr int kTileSide = kBinSide / 2, kTiles = kTileSide * kTileSide;
@@ -1548,6 +1546,7 @@ constexpr int kWideResolution = 97;                 // ... and so does one bin
 constexpr int kTileLdsValues = 48 * 48 * 4;         // the largest coarse level with F = 4: 72 KB
 constexpr int kBinBlock = 1024, kTileBlock = 512;
 constexpr int kMaxBinParts = 64;
+constexpr int kMostPieces = 6, kPieceBatch = 65536;   // fine levels: see tiled_level
 constexpr int kTileFlush = 3;                       // nodes a thread stores with their row lookups in flight together
 
 struct PackedTileArgs {
@@ -1847,6 +1846,50 @@ __device__ __forceinline__ void fine_tile(const TileLevel<F>& level, int tx, int
         }
 }
 
+// Most pieces a tile of a level of r x r nodes is cut into.
+template <int F> __device__ __forceinline__ int tile_pieces(int r) {
+    const int cap = kTileLdsValues / F;
+    const int width = (r - 1) / kTileSide + 2, across = min(width, cap), rows = max(1, cap / across);
+    return ((width + across - 1) / across) * ((width + rows - 1) / rows);
+}
+
+// Whether a level of r x r nodes is summed by tiles.  A tile of more nodes than LDS holds (past 1072 cells
+// with two features) is walked in pieces, each of which clears LDS, reads the tile's whole list and
+// looks for its nodes again: about 5 us a piece however small the batch, 12 us of 2^20 coordinates.
+// The atomics take 25 us of 65536 coordinates with two visible features, half with one, and less the
+// finer the plane, as less of it is visible.  Planes beside levels of 8 and 9 cells, us by pieces / by
+// atomics at 65536, 2^18 and 2^20 coordinates: 1290 cells F = 2 (2 pieces) 37/47, 62/123, 183/446; 2048 F = 2
+// (4, 54% visible) 55/35, 75/91, 181/327; 2048 F = 1 (2) 43/34, 63/75, 184/236; 3251 F = 2 (10, 19%) 85/28,
+// 131/57, 242/179; 5161 F = 1 (12, 7%) 89/25, 144/56, 297/177; 8192 F = 2 (57, 2%) 233/26, 421/56, 872/178.
+template <int F> __device__ __forceinline__ bool tiled_level(int r, int64_t n) {
+    const int pieces = tile_pieces<F>(r);
+    return pieces <= kMostPieces && static_cast<int64_t>(pieces * (pieces - 1)) * (kPieceBatch / F) <= n;
+}
+
+// A share of the sorted batch at a level that is not: straight to the gradient, as the pass without
+// scratch does.
+template <int F>
+__device__ __forceinline__ void scatter_level(const TileLevel<F>& level, int share) {
+    const PackedTileArgs& a = level.a;
+    const int64_t end = a.n * (share + 1) / kTiles;
+    for (int64_t j = a.n * share / kTiles + threadIdx.x; j < end; j += kTileBlock) {
+        const float4 entry = a.sorted[j];
+        const TileCorner at(make_float2(entry.x, entry.y), level.r);
+        const int cell = at.ix + at.iy * level.r;
+        float u[F];
+        const bool seen = level.visible(cell);
+        level.load(__float_as_uint(entry.z), u);
+        if (!seen) continue;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int row = node_row(a, level.d, (cell + (k & 1) + (k >> 1) * level.r) % level.points);
+#pragma unroll
+            for (int c = 0; c < F; ++c)
+                if (u[c] != 0.0f) atomicAdd(level.parameter(row, c), at.w[k] * u[c]);
+        }
+    }
+}
+
 template <int F>
 __device__ __forceinline__ void tile_level(const PackedTileArgs& a, const int32_t* d, int slot, double* acc) {
     const TileLevel<F> level(a, d);
@@ -1857,7 +1900,8 @@ __device__ __forceinline__ void tile_level(const PackedTileArgs& a, const int32_
     }
     // consecutive tiles on one XCD (a block's XCD is its index mod 8), so that they share its L2
     const int tile = (slot % kXcds) * (kTiles / kXcds) + slot / kXcds;
-    fine_tile(level, tile % kTileSide, tile / kTileSide, acc);
+    if (tiled_level<F>(level.r, a.n)) fine_tile(level, tile % kTileSide, tile / kTileSide, acc);
+    else scatter_level(level, tile);
 }
 
 __global__ __launch_bounds__(kTileBlock) void packed_tile_kernel(PackedTileArgs a) {

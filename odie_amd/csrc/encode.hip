@@ -1216,9 +1216,11 @@ ODIE_API int odie_packed_forward(const float* coords, int64_t n, const float* gr
 
 namespace odie {
 
-// Batches of this many coordinates go by spatial tiles when the caller gives scratch: faster than the
-// atomics at every size measured from here up (8, 16 and 20 levels, random and spatial order: 26
-// against 44 us, 39 against 86, 44 against 108 at 1024 coordinates).
+// Batches of this many coordinates go by spatial tiles when the caller gives scratch (the pass itself
+// sends planes too fine for its tiles to memory).  us, atomics / this, at 1024, 65536 and 2^20
+// coordinates: 16 levels up to 1020 cells, random 87/33, 213/56, 2728/403, in spatial order 85/33, 148/55,
+// 3272/435, in 3% of the side 106/32, 2032/415, 25486/6532; 16 levels up to 8192 cells 106/45, 259/80,
+// 3400/513, in 3% of the side 112/42, 1885/452, 24967/7762.  Smaller batches have not been measured.
 constexpr int64_t kTiledBatch = 1024;
 
 int packed_backward_internal(const float* coords, int64_t n, const uint16_t* upstream, int up_width,

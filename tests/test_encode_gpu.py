@@ -641,6 +641,50 @@ def test_packed_tiles_match_the_oracle_and_the_atomics(n, width, spread):
     check_gradient(atomics, bar, 'packed atomics, ' + spread)
 
 
+# Planes whose tiles take 2 pieces (1290 cells, F = 2), 3 (1200, F = 4) and 10 (3300, F = 2): summed by
+# tiles from 65536 and 98304 coordinates on, and never.
+FINE_PLANES = dict(resolutions=(8, 13, 49, 1290, 1200, 3300), dims=(1, 2, 1, 2, 4, 2), dense=3)
+
+
+@pytest.mark.parametrize('n', [2000, 65535, 65536, 98304])
+def test_packed_tiles_of_fine_planes(n):
+    layout = _packed_layout(26, **FINE_PLANES)
+    xy, up = synth.coordinates(26, n), synth.upstream(26, n, 12)
+    xy[:500] = 1.0 - np.float32(1e-4) * xy[:500]     # corners that wrap
+    host = {k: layout[k].numpy() for k in ('descriptors', 'node_bitmap', 'node_prefix', 'bitmap')}
+    expected, magnitude, counts = oracle.packed_backward(xy, up, host, layout['params'], counts=True)
+    got = _packed_gradient(layout, torch.from_numpy(xy).cuda(), torch.from_numpy(up).cuda(), packed_owner=0)
+    # an fp32 rounding per contribution added in memory, or per partial sum, and one for the sum
+    assert (np.abs(got.cpu().numpy().astype(np.float64) - expected) <= (counts + 33) * 2.0 ** -24 * magnitude).all()
+
+
+def test_packed_tiles_of_a_fine_plane_cost_no_more_than_the_atomics():
+    """6000 cells a side: the level goes to memory (32 pieces a tile took three times as long)."""
+    layout = _packed_layout(27, resolutions=(8, 13, 20, 6000), dims=(2, 2, 2, 2), dense=3)
+    n = 2048
+    d_xy = torch.from_numpy(synth.coordinates(27, n)).cuda()
+    d_up = torch.from_numpy(synth.upstream(27, n, 8)).cuda()
+    dev = {k: layout[k].cuda() for k in ('descriptors', 'node_bitmap', 'node_prefix', 'bitmap')}
+    lib, gradient = _lib.library(), torch.empty(layout['params'], device='cuda')
+    scratch = torch.empty(lib.odie_packed_backward_workspace(n, 8), dtype=torch.uint8, device='cuda')
+
+    def best(scratch):
+        times = []
+        for _ in range(10):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            _lib.check(lib.odie_packed_backward_scratch(
+                d_xy.data_ptr(), n, d_up.data_ptr(), 8, dev['descriptors'].data_ptr(), 4,
+                dev['node_bitmap'].data_ptr(), dev['node_prefix'].data_ptr(), dev['bitmap'].data_ptr(),
+                gradient.data_ptr(), layout['params'], _lib.ptr(scratch), 0 if scratch is None else scratch.numel(),
+                _lib.stream_of(gradient)))
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+    assert best(scratch) < 2 * best(None)
+
+
 def test_packed_tiles_column_scales_and_zero_upstream():
     """Columns 10^6 apart keep their own scale; an all-zero upstream clears the gradient."""
     layout = _packed_layout(22, **TILE_PLANES)
