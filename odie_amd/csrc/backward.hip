@@ -1283,13 +1283,17 @@ __global__ __launch_bounds__(kOwnerBlock) void owner_kernel(OwnerArgs a) {
 // owner does unsplit.
 __global__ __launch_bounds__(256) void split_reduce_kernel(OwnerArgs a) {
     const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
+    const int per_entry = __builtin_ctz(a.features);   // features: a power of two
     for (int e = blockIdx.y; e < a.experts; e += gridDim.y)
     for (int64_t x = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; x < a.partial_floats; x += stride) {
-        const uint32_t entry = static_cast<uint32_t>(x / a.features);
+        const uint32_t entry = static_cast<uint32_t>(x >> per_entry);
         int l = 0;
         while (l + 1 < a.n_levels && a.level[l + 1].offset <= entry) ++l;
         const int splits = l >= a.group ? a.splits[l] : a.group_splits;
         if (splits <= 1) continue;
+        int64_t base, stop;
+        expert_range(a.offsets, a.n, e, base, stop);
+        const uint32_t peak = a.peaks[(static_cast<int64_t>(e) * a.n_levels + l) * a.features + (x & (a.features - 1))];
         // eight independent loads in flight per round: the splits' partials are far apart
         const long long* column = a.partial64 + static_cast<int64_t>(e) * a.partial_floats + x;
         const int64_t step = static_cast<int64_t>(a.experts) * a.partial_floats;
@@ -1302,10 +1306,12 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(OwnerArgs a) {
 #pragma unroll
             for (int k = 0; k < 8; ++k) sum += v[k];
         }
-        for (; s < splits; ++s) sum += column[s * step];
-        int64_t base, stop;
-        expert_range(a.offsets, a.n, e, base, stop);
-        const uint32_t peak = a.peaks[(static_cast<int64_t>(e) * a.n_levels + l) * a.features + x % a.features];
+        for (; s < splits; s += 4) {
+            long long v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = s + k < splits ? column[(s + k) * step] : 0;
+            sum += (v[0] + v[1]) + (v[2] + v[3]);
+        }
         float v = unscaled(sum, column_shift(peak, stop - base));
         const int64_t i = static_cast<int64_t>(e) * a.expert_params + x;
         if (a.fused) {
@@ -2113,31 +2119,41 @@ int launch_owner_backward(const OwnerLaunch& in) {
         // its slice outweigh its adds (one step, 16 experts of 2^14 coordinates, 2^9 tables: shares
         // of 16384 / 8192 / 4096 / 2048 / 1024 403 / 289 / 241 / 217 / 216 us; 4 of 2^14, 2^10
         // tables: 267 / 177 / 140 / 126 / 148; 9 of 7800, 2^13 tables: 162 / 161 / 162 / 160 / 201).
+        // One round of workgroups, one to a CU, and the ways of the coarse group (about group + 1
+        // fine passes' work) and of the fine passes such that the longest item is shortest: a second
+        // round costs its clears and 16 bytes a value and split of partials more.  One step, all
+        // passes in 512 / passes ways, two rounds -> so: 4 experts, 2^20 coordinates, tables of 2^12
+        // 346 -> 304, 2^13 374 -> 323, 2^14 476 -> 365 us; 9 experts, 2^20, 2^11 333 -> 286; 16, 2^22, 2^9
+        // 741 -> 711.  One grid, 2^14-entry tables, forward and backward of 2^20 360 -> 260, 2^22 1247 -> 866;
+        // native step, 2^17 441 -> 235.  (group, fine) ways of 4 experts, 2^13: (20, 4) 309-323, (11, 11)
+        // 376, (11, 5) 362, (8, 4) 373, (24, 4) 346.
         // Otherwise only the coarse-group pass may be split:
         // it walks every coordinate through `group` fully landing levels, about group + 1 times
         // the work of a fine slice (measured: ~6x with 5 levels), and when that alone exceeds one
         // CU's share of the whole pass it would set the kernel's length, so it is cut into
         // pieces of about that share.
         const int64_t per_pass = static_cast<int64_t>(in.experts) * passes;
-        int splits = 1;
-        bool all = false;
         constexpr int64_t kLeastShare = 2048;
         if (per_pass < 128) {
-            const int64_t want = (512 + per_pass - 1) / per_pass;
-            const int64_t most = in.n / (static_cast<int64_t>(in.experts) * kLeastShare);
-            splits = static_cast<int>(want < most ? want : (most > 1 ? most : 1));
-            all = true;
+            const int64_t share = in.n / (static_cast<int64_t>(in.experts) * kLeastShare), most = share > 1 ? share : 1;
+            const int64_t items = kCus / in.experts, fine = group > 0 ? passes - 1 : passes;
+            double least = 0.0;
+            for (int64_t ways = 1; ways <= most; ++ways) {
+                const int64_t left = std::max<int64_t>(std::min(items - ways * fine, most), 1);
+                const double longest = std::max(fine > 0 ? 1.0 / ways : 0.0, group > 0 ? (group + 1.0) / left : 0.0);
+                if (ways > 1 && (longest >= least || ways * fine + (group > 0 ? 1 : 0) > items)) break;
+                least = longest;
+                for (int l = group; l < L; ++l) o.splits[l] = static_cast<int>(ways);
+                if (group > 0) group_splits = static_cast<int>(left);
+            }
         } else if (group > 0) {
             const double share = static_cast<double>(in.experts) * (passes + group) / kCus;   // fine-slice units
             if (group + 1 > share) {
                 const int64_t want = static_cast<int64_t>(std::ceil((group + 1) / (share > 1.0 ? share : 1.0)));
                 const int64_t most = in.n / (static_cast<int64_t>(in.experts) * 4096);
-                splits = static_cast<int>(want < most ? want : (most > 1 ? most : 1));
+                group_splits = static_cast<int>(want < most ? want : (most > 1 ? most : 1));
             }
         }
-        if (group > 0) group_splits = splits;
-        if (all)
-            for (int l = group; l < L; ++l) o.splits[l] = splits;
     }
     int items = group_splits;
     int heavy = group_splits;

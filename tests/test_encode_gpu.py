@@ -272,6 +272,17 @@ def test_unbanded_splits_are_exact(log2, experts, n):
         assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize('log2,experts,n', [(13, 4, 1 << 20), (14, 4, 1 << 18), (11, 9, 150001), (7, 1, 100000),
+                                            (9, 120, 1 << 19), (16, 2, 50000), (14, 15, 120000)])
+def test_unbanded_splits_of_one_round_are_exact(log2, experts, n):
+    """The group and the fine passes split in different ways (one pass alone, two ways left, no room for a
+    second way, the group alone split): the gradient equals the unsplit one bit for bit."""
+    levels, params, offsets, xy, up = _expert_batch(log2 + 3, log2, experts, n)
+    run = lambda: grid_backward(xy, up.half(), levels, 2, offsets=offsets, experts=experts, expert_params=params)
+    split = _tuned('banded', 0, 2, run)
+    assert torch.equal(split, _tuned('banded', 1, 2, lambda: _tuned('split_target', 1 << 30, 0, run)))
+
+
 def test_banded_owner_with_unordered_offsets():
     """Offsets that decrease somewhere make the expert ranges overlap: the band lists are not
     used and the fine passes walk the experts' index ranges, as the unbanded owner does."""
