@@ -827,6 +827,27 @@ def test_grid_encoding_with_its_handoff_equals_the_plain_pair(n, log2, levels, f
         assert torch.equal(module(xy), want)
 
 
+@pytest.mark.parametrize('n,log2,levels,features,dtype,formed', [
+    (65535, 14, 16, 2, torch.float16, False), (65536, 14, 16, 2, torch.float16, True),      # slice masks
+    (65536, 19, 16, 2, torch.float16, False), (196607, 19, 12, 4, torch.float32, False),    # band lists
+    (196608, 19, 16, 2, torch.float16, True), (200003, 19, 12, 4, torch.float32, True)])
+def test_grid_encoding_forms_its_handoff_where_it_pays(n, log2, levels, features, dtype, formed):
+    """A forward that no backward may follow does not pay for lists that a small batch's backward gains
+    little from; either way the pair is the plain one bit for bit."""
+    from odie_amd.encoding import GridEncoding
+    module = GridEncoding(dict(n_levels=levels, n_features_per_level=features, log2_hashmap_size=log2,
+                               base_resolution=16, per_level_scale=1.38), dtype=dtype)
+    with torch.no_grad():
+        module.params.copy_(torch.from_numpy(synth.table(33, module.n_params, -1.0, 1.0, name='enc')))
+    xy = torch.from_numpy(synth.coordinates(33, n)).cuda()
+    up = torch.from_numpy(synth.upstream(33, n, module.n_output_dims)).cuda().to(dtype)
+    out = module(xy)
+    assert (out.grad_fn.saved_tensors[1] is not None) == formed
+    assert torch.equal(out.detach(), grid_forward(xy, module.params.detach().to(dtype), module.levels, features))
+    got, = torch.autograd.grad(out, module.params, up)
+    assert torch.equal(got, grid_backward(xy, up, module.levels, features, expert_params=module.n_params))
+
+
 def test_without_memory_for_optional_scratch(monkeypatch):
     """No room for the tiles' scratch or the handoff: the passes that need none run instead."""
     from odie_amd.encoding import GridEncoding
