@@ -132,7 +132,9 @@ class GreedySelection:
         """Move the state to where most of the choices have been made (odie_selection_relax,
         odie_selection_bulk).  A pass that raised no level ends the relaxation."""
         need = int(lib.odie_selection_bulk_workspace(self.points))
-        workspace = torch.empty(need, dtype=torch.uint8, device=self.scores.device)
+        workspace = _lib.optional_bytes(need, self.scores.device)
+        if workspace is None:   # no room for it: every choice in its turn
+            return
         passes, launched = 6, 0
         while launched < 256:
             flags = torch.zeros(passes, dtype=torch.int64, device=self.scores.device)

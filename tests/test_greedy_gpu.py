@@ -113,6 +113,21 @@ def test_bulk_start_equals_one_choice_at_a_time(kind, resolution):
             assert torch.equal(got[0], selected) and torch.equal(got[1], nodes), what
 
 
+def test_without_memory_for_the_bulk_start(monkeypatch):
+    """No room for the head start's workspace: every choice is made in its turn."""
+    scores = torch.from_numpy(_bulk_scores('uniform', 65)).cuda()
+    want = select_device(scores, 65, 512)
+    empty = torch.empty
+
+    def refusing(*size, **options):
+        if options.get('dtype') == torch.uint8 and size and isinstance(size[0], int) and size[0] > 8 * 4225:
+            raise torch.cuda.OutOfMemoryError('no room')
+        return empty(*size, **options)
+    monkeypatch.setattr(torch, 'empty', refusing)
+    got = select_device(scores, 65, 512)
+    assert got[2] == want[2] and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 def test_bulk_start_against_the_oracle():
     values = _scores(17, 150 * 150, False)
     selected, nodes, iterations = oracle.select_benefit_cost(values, 150, 4000)
