@@ -338,6 +338,8 @@ def decode_rows(raw, gate, decoder, visible=None, columns=None):
     """The heads on raw features [N, sum F] fp16: columns padded with ones to the decoder's
     width, gated per level when there is a gate, decoded; RGB fp32 [N, 3].  Rows already of the
     decoder's width are read as they are; of those, the columns past `columns` count as ones."""
+    if raw.ndim != 2:
+        raise ValueError('decoder input must be CUDA fp16 [n, %d]' % decoder.width)
     if raw.shape[1] != decoder.width or raw.dtype != torch.float16 or raw.data_ptr() % 16:
         rows = torch.ones((raw.shape[0], decoder.width), dtype=torch.float16, device=raw.device)
         rows[:, :raw.shape[1]] = raw
@@ -396,6 +398,8 @@ class PackedXYPlanes(PackedPlanes):
             _check_query(coordinates)
             coordinates = coordinates.contiguous()
             n, width = coordinates.shape[0], self.decoder.width
+            if self.input_width > width:
+                raise ValueError('the planes have %d features, the decoder %d inputs' % (self.input_width, width))
             raw = torch.empty((n, width), dtype=torch.float16, device=coordinates.device)
             visible = torch.empty((n, self.n_levels), dtype=torch.uint8, device=coordinates.device)
             if self.grid.dtype != torch.float32 or self.grid.ndim != 1:

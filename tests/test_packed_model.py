@@ -7,7 +7,8 @@ import torch
 
 from odie_amd import synth
 from odie_amd.hash_grid import HashGrid
-from odie_amd.model import PackedXYPlanes, build_model
+from odie_amd.decoder import Decoder
+from odie_amd.model import PackedXYPlanes, build_model, decode_rows
 
 RESOLUTIONS = [4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 40, 48, 64, 80, 96, 128]
 
@@ -143,6 +144,23 @@ def test_native_optimizer_trains_a_packed_model():
     assert not torch.equal(model.decoder.params, decoder)
     assert not torch.equal(model.gate.params, gate)
     assert not torch.equal(model.forward(xy), before)
+
+
+@pytest.mark.gpu
+def test_rows_the_heads_do_not_take_are_refused():
+    """A decoder narrower than the planes' features, and rows that are not a matrix."""
+    supports, dims, caps = _inputs(9)
+    model = PackedXYPlanes(_config(**_head_sizes(dims)), supports, dims, caps)
+    xy = torch.rand((5, 2), device='cuda')
+    gate, decoder = model.gate, model.decoder
+    model.gate, model.decoder = None, Decoder(seed=1, width=16)
+    with pytest.raises((ValueError, RuntimeError)):
+        model(xy)
+    model.gate, model.decoder = gate, decoder
+    rows = torch.rand((5, decoder.width, 2), device='cuda').half()
+    with pytest.raises((ValueError, RuntimeError)):
+        decode_rows(rows, None, decoder)
+    assert model(xy).shape == (5, 3)
 
 
 def test_host_coordinates_are_refused():
