@@ -384,8 +384,17 @@ template <bool FAST> __global__ __launch_bounds__(kReconBlock) void score_cells_
 // a wave per cell, 3.0 with four waves, 2.2 with the fast encode and seven waves (two workgroups per
 // CU, so that 1024 cells are two full rounds; four waves and one step between barriers 2.6, eleven
 // waves 2.5 - 2.7).  Now bound by VALU issue (1.7 ms of it) and the gathers' address path (TA busy
-// 73%).  Up to a cell per CU: fifteen waves, one workgroup per CU (2.3 ms at 1024 cells).
+// 73%).  Up to a cell per CU: fifteen waves, one workgroup per CU.
+//
+// Where the lines lie, us by one wave / seven waves a cell: 1024^2 pixels in cells of 24^2 84/130, 31^2
+// 130/76, 32^2 (1024 cells) 118/69, 64^2 437/74; 4096^2 in 16^2 702/2154, 31^2 721/838, 32^2 (16384
+// cells) 671/833, 40^2 (10609) 734/987, 48^2 (7396) 779/763, 64^2 724/654, 128^2 1788/573; 8192^2 in 32^2
+// 2504/3272, 64^2 (16384) 2556/2503, 256^2 7084/2131.  So small cells need many pixels to be worth a
+// workgroup, and where there are enough cells to fill the chip with waves of one, four times as many.
+// Fifteen / seven waves: 4096^2 in 256 cells 566/744, 196 833/1063, 64 2185/2935, 1 143.1/191.3 ms; 8192^2
+// in 256 2148/2901, 1024 2193/2130; 1024^2 in 256 65/74, 484 98/74.
 constexpr int64_t kLargeCell = 1024;   // pixels per cell from which a cell gets several waves
+constexpr int64_t kManyCells = 8192;   // more cells: from 4 kLargeCell on
 constexpr int kScoreSteps = 4;         // 32 pixels per wave, this many times between two barriers
 
 template <bool FAST, int WAVES>
@@ -556,7 +565,8 @@ ODIE_API int odie_reconstruct_scores(int width, int height, int regions_x, int r
     ScoreArgs sc{target, resolution, xb, yb, totals, squares};
     const int64_t cells = static_cast<int64_t>(resolution) * resolution;
     const hipStream_t st = as_stream(stream);
-    if (static_cast<int64_t>(width) * height / cells >= kLargeCell) {
+    const int64_t large = cells > kManyCells ? 4 * kLargeCell : kLargeCell;
+    if (static_cast<int64_t>(width) * height / cells >= large) {
         const uint32_t grid = static_cast<uint32_t>(cells < 65536 ? cells : 65536);
         const bool few = cells <= kCus;
         if (fast && few) score_large_cells_kernel<true, 15><<<grid, 1024, 0, st>>>(a, bounds, sc);

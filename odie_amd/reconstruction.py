@@ -48,7 +48,7 @@ def score_image(grid, decoder_half, target, shape, regions, *, resolution=None, 
     """Reconstruct the whole image and score it: returns ({'mse', 'psnr_db'}, DeviceScores).
     target: CUDA uint8 [H*W, 3].  Cells are the native geometry cells at `resolution`, or
     uniform tiles of `tile` pixels (DeviceScores).  fused: one odie_reconstruct_scores launch
-    (a wave per cell, no prediction in memory unless `prediction` [H*W, 3] is given); otherwise
+    (one or several waves per cell, no prediction in memory unless `prediction` [H*W, 3] is given); otherwise
     batches of `batch` pixels through odie_reconstruct and score_chunk with the reference's torch
     mse."""
     height, width = shape
