@@ -11,7 +11,7 @@ import pytest
 import torch
 
 import oracle
-from odie_amd import synth
+from odie_amd import _lib, synth
 from odie_amd.decoder import Decoder
 from odie_amd.experts import ExpertGrid, route
 from odie_amd.gpu_residual import DeviceScores
@@ -126,8 +126,7 @@ def test_device_image_on_the_gpu_equals_numpy():
     ((40, 40), None, 7),         # small cells, one wave each, chunks across row ends
 ])
 def test_scores_of_cells_of_every_size(shape, resolution, tile):
-    """Cells on both sides of the large-cell rule against the oracle's sequential totals, bit for bit,
-    continuing totals that are not zero."""
+    """Cells on both sides of the large-cell rule against the oracle's sequential totals, bit for bit."""
     regions = (5, 3)
     grid, decoder = _model(6, regions[0] * regions[1])
     image = synth.image(8, shape[1], shape[0]).reshape(-1, 3)
@@ -180,3 +179,80 @@ def test_infinite_predictions_keep_their_scores():
     assert np.array_equal(np.isnan(got), np.isnan(expected)) and np.array_equal(np.isinf(got), np.isinf(expected))
     finite = np.isfinite(expected)
     assert np.array_equal(got[finite], expected[finite])
+
+
+# Past 2^22 cells the reconstruction takes the general geometry in place of its fast encode.
+GENERAL = dict(n_levels=16, base_resolution=40, log2_hashmap_size=6, per_level_scale=2.3, n_features_per_level=2)
+# A wave a cell, for few pixels and for many cells; several waves a cell, at most and more cells than CUs.
+CELL_CLASSES = [((101, 77), 9, None), ((2912, 2912), None, 32), ((330, 330), None, 33), ((640, 640), None, 32)]
+
+
+def _encoded(encoding, seed, experts):
+    grid = ExpertGrid(encoding, experts)
+    grid.table.copy_(torch.from_numpy(synth.table(seed, grid.table.numel(), -1.0, 1.0, name='general')).half())
+    return grid, Decoder(seed=seed)
+
+
+def _fused_scores(grid, decoder, target, shape, regions, scores):
+    """odie_reconstruct_scores into scores.totals as they stand; the squares per cell."""
+    squares = torch.zeros_like(scores.totals)
+    xb, yb = scores.xb.to(torch.int32).contiguous(), scores.yb.to(torch.int32).contiguous()
+    _lib.check(_lib.library().odie_reconstruct_scores(
+        shape[1], shape[0], regions[0], regions[1], None, grid.experts, grid.table.data_ptr(), grid.expert_params,
+        grid.levels, len(grid.levels), decoder.half.data_ptr(), target.data_ptr(), scores.resolution, xb.data_ptr(),
+        yb.data_ptr(), scores.totals.data_ptr(), squares.data_ptr(), None, _lib.stream_of(target)))
+    return squares
+
+
+def test_general_geometry_reconstruction():
+    shape, regions = (77, 201), (4, 3)
+    grid, decoder = _encoded(GENERAL, 11, 12)
+    assert max(level.resolution for level in grid.levels) >= 1 << 22
+    n = shape[0] * shape[1]
+    features = torch.empty((n, 32), dtype=torch.float16, device='cuda')
+    output = torch.empty((n, 16), dtype=torch.float16, device='cuda')
+    reconstruct(grid, decoder.half, shape, regions, 0, n, features=features, output=output)
+    want_features, want_output = _composed(grid, decoder, shape, regions, 0, n)
+    assert np.array_equal(_bits(features), _bits(want_features))
+    assert np.array_equal(_bits(output), _bits(want_output))
+
+
+@pytest.mark.parametrize('encoding', [ENCODING, GENERAL], ids=['fast', 'general'])
+@pytest.mark.parametrize('shape,resolution,tile', CELL_CLASSES)
+def test_scores_continue_totals_in_every_cell_class(shape, resolution, tile, encoding):
+    """Totals that are not zero are carried on in raster order, bit for bit, whichever kernel scores the
+    cells and whichever geometry encodes."""
+    regions = (5, 3)
+    grid, decoder = _encoded(encoding, 12, 15)
+    image = synth.image(13, shape[1], shape[0]).reshape(-1, 3)
+    target = torch.from_numpy(image).cuda()
+    scores = DeviceScores(shape, resolution=resolution, tile=tile)
+    start = synth.uniform(14, 'totals', scores.resolution ** 2).astype(np.float64) * 1e-3 + 0.1
+    scores.totals.copy_(torch.from_numpy(start))
+    squares = _fused_scores(grid, decoder, target, shape, regions, scores)
+    prediction = reconstruct(grid, decoder.half, shape, regions, 0, len(image)).cpu().numpy()
+    expected = oracle.residual(prediction, image, shape[1], scores.resolution, scores.xb.cpu().numpy(),
+                               scores.yb.cpu().numpy(), totals=start.copy())
+    assert np.array_equal(scores.totals.cpu().numpy().view(np.uint64), expected.view(np.uint64))
+    error = np.square(prediction - image.astype(np.float32) * np.float32(1 / 255)).astype(np.float64).sum()
+    assert float(squares.sum()) == pytest.approx(error, rel=1e-10)   # fp64 sums in another order
+
+
+@pytest.mark.parametrize('encoding', [ENCODING, GENERAL], ids=['fast', 'general'])
+@pytest.mark.parametrize('shape,resolution,tile', CELL_CLASSES)
+def test_fused_scores_of_infinite_predictions(shape, resolution, tile, encoding):
+    """An expert whose decoder overflows fp16: its cells' infinite and NaN totals, and the others' finite
+    ones, as the streamed pass forms them."""
+    regions = (5, 3)
+    grid, decoder = _encoded(encoding, 15, 15)
+    grid.table.view(15, -1)[4] = 6e4
+    target = torch.from_numpy(synth.image(16, shape[1], shape[0]).reshape(-1, 3)).cuda()
+    fused, streamed = (DeviceScores(shape, resolution=resolution, tile=tile) for _ in range(2))
+    _fused_scores(grid, decoder, target, shape, regions, fused)
+    prediction = reconstruct(grid, decoder.half, shape, regions, 0, shape[0] * shape[1])
+    streamed.add(prediction, target, 0)
+    got, want = fused.totals.cpu().numpy(), streamed.totals.cpu().numpy()
+    finite = np.isfinite(want)
+    assert finite.any() and not finite.all()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    assert np.array_equal(got[finite].view(np.uint64), want[finite].view(np.uint64))
