@@ -89,23 +89,6 @@ __device__ inline int64_t source_row(const TransposeArgs& a, bool by_list, int64
     return by_list && i >= lo && i < hi ? static_cast<int64_t>(a.list[i]) : i;
 }
 
-// Maximum of two |upstream| records; NaN wins, so the owner pass sees a non-finite bound.
-__device__ inline float nan_max(float a, float b) { return (b > a || b != b) ? b : a; }
-
-// Record q of the block (rows q*128.. of its 1024) is waves 2*(q%2) and 2*(q%2)+1 of pass q/2;
-// `waves` holds `stride` column maxima per wave, of which the first `columns` are used.
-__device__ inline void write_records(const TransposeArgs& a, const float* waves, int stride, int columns) {
-    constexpr int kRecords = kTransposeRows / kMaxRows;
-    for (int t = threadIdx.x; t < kRecords * columns; t += kTransposeBlock) {
-        const int q = t / columns, j = t % columns;
-        const int64_t record = static_cast<int64_t>(blockIdx.x) * kRecords + q;
-        if (record * kMaxRows >= a.n) continue;
-        const float* pass = waves + (q / 2) * (kTransposeBlock / 64) * stride;
-        const int w = 2 * (q % 2);
-        a.blockmax[record * columns + j] = nan_max(pass[w * stride + j], pass[(w + 1) * stride + j]);
-    }
-}
-
 // Maxima of N magnitudes (N a power of two; unsigned bit patterns: NaN above infinity above every
 // finite value) over the wave's 64 lanes, as a tree that halves the values a lane holds while it
 // doubles the lanes they cover: N + N/2 + ... exchanges in place of 6 N.  Each lane stores what it ends

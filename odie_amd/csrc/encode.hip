@@ -497,10 +497,6 @@ struct PackedArgs {
     int zero_off;        // levels >= active are evaluated and multiplied by 0 (else 0 outright)
 };
 
-__device__ inline int64_t plane_param(const PackedArgs& a, const int32_t* d, int cell, int k, int c) {
-    return packed_param(d, a.node_bitmap, a.prefix, a.params, cell, k, c);
-}
-
 // The packed query.  Bound by latency: per level a coordinate takes its cell's bit, its corners' rank
 // words and then their parameters, three dependent rounds of loads.  So a workgroup takes 64
 // coordinates and its four waves a quarter of the levels each (the levels stay uniform in a wave), a

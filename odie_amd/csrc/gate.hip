@@ -176,10 +176,6 @@ __device__ inline float gate_value(float z, int level, const GateArgs& a) {
     return 1.0f / (1.0f + expf(-z));
 }
 
-__device__ inline float visible_of(const GateArgs& a, int64_t row, int level) {
-    return a.visible ? static_cast<float>(a.visible[row * a.levels + level]) : 1.0f;
-}
-
 // A lane's four consecutive levels 8q + 4g .. + 3 of a row of L values: one load or store where rows
 // of L values keep the alignment (L a multiple of 4), else one by one; levels past L are 0.
 __device__ inline void visible4(const GateArgs& a, int64_t row, bool valid, int first, float out[4]) {

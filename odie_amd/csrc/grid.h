@@ -126,10 +126,8 @@ __device__ inline void plane_geometry(float x, float y, int r, int& cell, float 
     w[3] = fx * fy;
 }
 
-// Parameter of feature c of corner k of `cell`: node (cell + k%2 + (k/2) R) mod points, its row
-// (the node itself, or its rank among the stored nodes: word prefix + popcount below it),
-// plane offset + row * features + c, clamped into the parameters.
-// Row of corner k of `cell` (the first half of packed_param; the same for every feature).
+// Row of corner k of `cell`, the same for every feature: node (cell + k%2 + (k/2) R) mod points itself,
+// or its rank among the stored nodes (word prefix + popcount below it).
 __device__ inline int packed_row(const int32_t* d, const uint64_t* node_bitmap, const int32_t* prefix, int cell,
                                  int k) {
     const int node = (cell + (k & 1) + (k >> 1) * d[0]) % d[1];
@@ -139,19 +137,11 @@ __device__ inline int packed_row(const int32_t* d, const uint64_t* node_bitmap, 
     return prefix[word] + __popcll(node_bitmap[word] & mask);
 }
 
-// Parameter of feature c of a corner in row `row`, clamped into the parameters.
+// Parameter of feature c of a corner in row `row`: plane offset + row * features + c, clamped into the
+// parameters.
 __device__ inline int64_t packed_at(const int32_t* d, int64_t params, int row, int c) {
     const int64_t p = static_cast<int64_t>(d[2]) + static_cast<int64_t>(row) * d[5] + c;
     return p < 0 ? 0 : (p >= params ? params - 1 : p);
-}
-
-__device__ inline int64_t packed_param(const int32_t* d, const uint64_t* node_bitmap, const int32_t* prefix,
-                                       int64_t params, int cell, int k, int c) {
-    return packed_at(d, params, packed_row(d, node_bitmap, prefix, cell, k), c);
-}
-
-__device__ inline bool cell_visible(const int32_t* d, const uint8_t* bitmap, int cell) {
-    return (bitmap[d[4] + (cell >> 3)] >> (cell & 7)) & 1;
 }
 
 // Host: device rows of an odie_grid_level table (levels contiguous from entry 0); entries
