@@ -696,6 +696,30 @@ def test_packed_tiles_of_a_fine_plane_cost_no_more_than_the_atomics():
     assert best(scratch) < 2 * best(None)
 
 
+def _planes_of_features(features, dense):
+    """A layout's descriptors stretched to another feature count than layouts have (1, 2 or 4)."""
+    layout = _packed_layout(28, resolutions=(8, 13, 20, 130, 64), dims=(1,) * 5, dense=dense)
+    layout['descriptors'][:, [2, 5, 6]] *= features
+    return layout, layout['params'] * features, 5 * features
+
+
+@pytest.mark.parametrize('features', [3, 6, 8])
+@pytest.mark.parametrize('n,dense', [(1000, 5), (5000, 3)])
+def test_packed_forward_of_any_feature_count(features, n, dense):
+    """Bit for bit, the last feature of the last node among them."""
+    from odie_amd.model import packed_forward
+    layout, params, width = _planes_of_features(features, dense)
+    xy = synth.coordinates(28, n)
+    xy[-200:] = 1.0 - np.float32(1e-5) * xy[-200:]
+    grid = synth.table(28, params, -0.5, 0.5)
+    host = {k: layout[k].numpy() for k in ('descriptors', 'node_bitmap', 'node_prefix', 'bitmap')}
+    dev = [layout[k].cuda() for k in ('descriptors', 'node_bitmap', 'node_prefix', 'bitmap')]
+    out, visible = packed_forward(torch.from_numpy(xy).cuda(), torch.from_numpy(grid).cuda(), *dev, width)
+    want, seen = oracle.packed_forward(xy, grid, host, width)
+    assert np.array_equal(out.cpu().numpy().view(np.uint16), want.view(np.uint16))
+    assert np.array_equal(visible.cpu().numpy(), seen)
+
+
 def test_packed_tiles_column_scales_and_zero_upstream():
     """Columns 10^6 apart keep their own scale; an all-zero upstream clears the gradient."""
     layout = _packed_layout(22, **TILE_PLANES)
