@@ -1855,42 +1855,44 @@ template <int F> __device__ __forceinline__ bool tiled_level(int r, int64_t n) {
     return pieces <= kMostPieces && static_cast<int64_t>(pieces * (pieces - 1)) * (kPieceBatch / F) <= n;
 }
 
-// A share of the sorted batch at a level that is not: straight to the gradient, as the pass without
-// scratch does.
-template <int F>
-__device__ __forceinline__ void scatter_level(const TileLevel<F>& level, int share) {
-    const PackedTileArgs& a = level.a;
+// A share of the sorted batch at a level that is not, or whose feature count has no tiles: straight to
+// the gradient, as the pass without scratch does.
+__device__ __forceinline__ void scatter_level(const PackedTileArgs& a, const int32_t* d, int share) {
+    const int features = min(d[5], a.width - d[6]);
     const int64_t end = a.n * (share + 1) / kTiles;
     for (int64_t j = a.n * share / kTiles + threadIdx.x; j < end; j += kTileBlock) {
         const float4 entry = a.sorted[j];
-        const TileCorner at(make_float2(entry.x, entry.y), level.r);
-        const int cell = at.ix + at.iy * level.r;
-        float u[F];
-        const bool seen = level.visible(cell);
-        level.load(__float_as_uint(entry.z), u);
-        if (!seen) continue;
+        const TileCorner at(make_float2(entry.x, entry.y), d[0]);
+        const int cell = at.ix + at.iy * d[0];
+        if (!((a.bitmap[d[4] + (cell >> 3)] >> (cell & 7)) & 1)) continue;
+        int row[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int row = node_row(a, level.d, (cell + (k & 1) + (k >> 1) * level.r) % level.points);
+        for (int k = 0; k < 4; ++k) row[k] = node_row(a, d, (cell + (k & 1) + (k >> 1) * d[0]) % d[1]);
+        const uint16_t* upstream = a.upstream + static_cast<int64_t>(__float_as_uint(entry.z)) * a.width + d[6];
+        for (int c = 0; c < features; ++c) {
+            const float u = __half2float(bits_to_half(upstream[c]));
+            if (u == 0.0f) continue;
 #pragma unroll
-            for (int c = 0; c < F; ++c)
-                if (u[c] != 0.0f) atomicAdd(level.parameter(row, c), at.w[k] * u[c]);
+            for (int k = 0; k < 4; ++k) atomicAdd(a.gradient + packed_at(d, a.params, row[k], c), at.w[k] * u);
         }
     }
 }
+
+// Consecutive tiles on one XCD (a block's XCD is its index mod 8), so that they share its L2.
+__device__ __forceinline__ int tile_of_slot(int slot) { return (slot % kXcds) * (kTiles / kXcds) + slot / kXcds; }
 
 template <int F>
 __device__ __forceinline__ void tile_level(const PackedTileArgs& a, const int32_t* d, int slot, double* acc) {
     const TileLevel<F> level(a, d);
     if (level.used == 0) return;
-    if (level.r < kFineResolution) {
+    const int tile = tile_of_slot(slot);
+    if (level.r < kFineResolution && level.points <= kTileLdsValues / F) {
         if (slot < a.splits) coarse_level(level, slot, acc);
-        return;
+    } else if (level.r >= kFineResolution && tiled_level<F>(level.r, a.n)) {
+        fine_tile(level, tile % kTileSide, tile / kTileSide, acc);
+    } else {
+        scatter_level(a, d, tile);
     }
-    // consecutive tiles on one XCD (a block's XCD is its index mod 8), so that they share its L2
-    const int tile = (slot % kXcds) * (kTiles / kXcds) + slot / kXcds;
-    if (tiled_level<F>(level.r, a.n)) fine_tile(level, tile % kTileSide, tile / kTileSide, acc);
-    else scatter_level(level, tile);
 }
 
 __global__ __launch_bounds__(kTileBlock) void packed_tile_kernel(PackedTileArgs a) {
@@ -1901,7 +1903,7 @@ __global__ __launch_bounds__(kTileBlock) void packed_tile_kernel(PackedTileArgs 
         case 1: tile_level<1>(a, d, slot, sums); break;
         case 2: tile_level<2>(a, d, slot, sums); break;
         case 4: tile_level<4>(a, d, slot, sums); break;
-        default: break;
+        default: scatter_level(a, d, tile_of_slot(slot)); break;
     }
 }
 

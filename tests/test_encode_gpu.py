@@ -720,6 +720,21 @@ def test_packed_forward_of_any_feature_count(features, n, dense):
     assert np.array_equal(visible.cpu().numpy(), seen)
 
 
+@pytest.mark.parametrize('features', [3, 6, 8])
+@pytest.mark.parametrize('n,dense', [(1000, 5), (5000, 3), (5000, 5)])
+def test_packed_backward_of_any_feature_count(features, n, dense):
+    """With scratch and without: levels whose feature count has no tiles go to memory."""
+    layout, params, width = _planes_of_features(features, dense)
+    xy, up = synth.coordinates(28, n), synth.upstream(28, n, width)
+    xy[-200:] = 1.0 - np.float32(1e-5) * xy[-200:]
+    host = {k: layout[k].numpy() for k in ('descriptors', 'node_bitmap', 'node_prefix', 'bitmap')}
+    expected, magnitude, counts = oracle.packed_backward(xy, up, host, params, counts=True)
+    got = _packed_gradient(dict(layout, params=params), torch.from_numpy(xy).cuda(), torch.from_numpy(up).cuda(),
+                           packed_owner=0)
+    # an fp32 rounding per contribution added in memory, and one for the sum
+    assert (np.abs(got.cpu().numpy() - expected) <= (counts + 1) * 2.0 ** -24 * magnitude).all()
+
+
 def test_packed_tiles_column_scales_and_zero_upstream():
     """Columns 10^6 apart keep their own scale; an all-zero upstream clears the gradient."""
     layout = _packed_layout(22, **TILE_PLANES)
