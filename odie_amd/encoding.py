@@ -105,8 +105,7 @@ def _check_handoff(handoff):
         raise ValueError('handoff must be a contiguous CUDA uint8 tensor')
 
 
-# A training forward forms the handoff from these many coordinates on: slice masks, and band lists.
-HANDOFF_BATCH, LIST_BATCH = 65536, 3 << 16
+HANDOFF_BATCH = 3 << 16
 
 
 class _GridEncode(torch.autograd.Function):
@@ -115,21 +114,19 @@ class _GridEncode(torch.autograd.Function):
         table = params if module.dtype == torch.float32 else params.to(module.dtype)
         # what the backward would form again in passes of its own (its band lists or slice masks)
         # comes from the forward, which walks the lists itself; like the coordinates it is saved
-        # for this backward alone.  No backward may come, so a line lies where what the pair gains
-        # reaches what the forward pays.  Small batches are bound by the host: 4096 coordinates 118 ->
-        # 128 us a pair with masks; from 65536 on they cost the forward 0 to 3 us and save the pair 1
-        # to 12.  Lists (2^19-entry tables; fp16 with two features, fp32 with four), forward / pair, us:
+        # for this backward alone.  No backward may come, so the line lies where what the pair gains
+        # reaches what the forward pays.  Below it masks save the pair 1 to 3 us and cost the host as
+        # much (4096 coordinates 118 -> 128 us with them); above it 2 to 40, for at most 5 of the forward.
+        # Lists (2^19-entry tables; fp16 with two features, fp32 with four), forward / pair, us:
         # 65536 27.7 -> 63.4 / 166 -> 163 and 19.4 -> 52.3 / 227 -> 224, 131072 32.8 -> 64.8 / 170 -> 165 and
         # 28.4 -> 56.9 / 240 -> 232, 200003 42.6 -> 67.4 / 182 -> 172 and 52.4 -> 65.5 / 272 -> 250, 300007
         # 54.7 -> 70.7 / 207 -> 187 and 66.1 -> 72.1 / 301 -> 269, 2^20 149 -> 116 / 424 -> 358 and 216 -> 135 /
         # 612 -> 500.
         size = 0
         if train and coords.ndim == 2 and coords.shape[0] >= HANDOFF_BATCH:
-            # with the forward's scratch, which only lists take: streams stay independent
-            plan = (coords.shape[0], 1, module.n_params, module.levels, len(module.levels), module.features)
-            size = max(_lib.library().odie_grid_handoff_own_bytes(*plan), 0)
-            if coords.shape[0] < LIST_BATCH and size > _lib.library().odie_grid_handoff_bytes(*plan):
-                size = 0
+            # with the forward's scratch: streams stay independent
+            size = max(_lib.library().odie_grid_handoff_own_bytes(coords.shape[0], 1, module.n_params, module.levels,
+                                                                  len(module.levels), module.features), 0)
         handoff = _lib.optional_bytes(size, coords.device)
         ctx.save_for_backward(coords, handoff)
         ctx.module = module

@@ -867,12 +867,13 @@ def test_grid_encoding_with_its_handoff_equals_the_plain_pair(n, log2, levels, f
 
 
 @pytest.mark.parametrize('n,log2,levels,features,dtype,formed', [
-    (65535, 14, 16, 2, torch.float16, False), (65536, 14, 16, 2, torch.float16, True),      # slice masks
+    (196607, 14, 16, 2, torch.float16, False), (196608, 14, 16, 2, torch.float16, True),    # slice masks
     (65536, 19, 16, 2, torch.float16, False), (196607, 19, 12, 4, torch.float32, False),    # band lists
     (196608, 19, 16, 2, torch.float16, True), (200003, 19, 12, 4, torch.float32, True)])
-def test_grid_encoding_forms_its_handoff_where_it_pays(n, log2, levels, features, dtype, formed):
+def test_grid_encoding_forms_its_handoff_where_it_pays(n, log2, levels, features, dtype, formed, monkeypatch):
     """A forward that no backward may follow does not pay for lists that a small batch's backward gains
-    little from; either way the pair is the plain one bit for bit."""
+    little from; either way the pair is the plain one bit for bit, also on a second backward, after a
+    tuning change in between, and where there is no memory for the handoff."""
     from odie_amd.encoding import GridEncoding
     module = GridEncoding(dict(n_levels=levels, n_features_per_level=features, log2_hashmap_size=log2,
                                base_resolution=16, per_level_scale=1.38), dtype=dtype)
@@ -883,8 +884,17 @@ def test_grid_encoding_forms_its_handoff_where_it_pays(n, log2, levels, features
     out = module(xy)
     assert (out.grad_fn.saved_tensors[1] is not None) == formed
     assert torch.equal(out.detach(), grid_forward(xy, module.params.detach().to(dtype), module.levels, features))
-    got, = torch.autograd.grad(out, module.params, up)
-    assert torch.equal(got, grid_backward(xy, up, module.levels, features, expert_params=module.n_params))
+    want = grid_backward(xy, up, module.levels, features, expert_params=module.n_params)
+    for last in (False, True):
+        got, = torch.autograd.grad(out, module.params, up, retain_graph=not last)
+        assert torch.equal(got, want)
+    out = module(xy)
+    changed = _tuned('banded', 0, 2, lambda: [torch.autograd.grad(out, module.params, up)[0], grid_backward(
+        xy, up, module.levels, features, expert_params=module.n_params)])
+    assert torch.equal(*changed)
+    monkeypatch.setattr(_lib, 'optional_bytes', lambda size, device: None)
+    got, = torch.autograd.grad(module(xy), module.params, up)
+    assert torch.equal(got, want)
 
 
 def test_without_memory_for_optional_scratch(monkeypatch):
