@@ -1843,7 +1843,7 @@ template <int F> __device__ __forceinline__ int tile_pieces(int r) {
     return ((width + across - 1) / across) * ((width + rows - 1) / rows);
 }
 
-// Whether a level of r x r nodes is summed by tiles.  A tile of more nodes than LDS holds (past 1072 cells
+// Whether a level of r x r nodes is summed by tiles.  A tile of more nodes than LDS holds (past 1056 cells
 // with two features) is walked in pieces, each of which clears LDS, reads the tile's whole list and
 // looks for its nodes again: about 5 us a piece however small the batch, 12 us of 2^20 coordinates.
 // The atomics take 25 us of 65536 coordinates with two visible features, half with one, and less the
