@@ -579,7 +579,7 @@ __global__ __launch_bounds__(kBlock) void packed_forward_kernel(PackedArgs a) {
             const int l = l0 + 4 * q;
             if (l >= a.levels) continue;
             const int32_t* d = a.desc + 8 * l;
-            const bool even = grid_even && d[2] % 2 == 0 && d[5] % 2 == 0;
+            const bool even = grid_even && ((d[2] | d[5]) & 1) == 0;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 if (!d[7]) row[q][k] += __popcll(word[q][k]);
@@ -600,7 +600,7 @@ __global__ __launch_bounds__(kBlock) void packed_forward_kernel(PackedArgs a) {
             const pair weight[4] = {(pair){w01.x, w01.x}, (pair){w01.y, w01.y}, (pair){w23.x, w23.x}, (pair){w23.y, w23.y}};
             for (int c = 0; c < d[5]; c += 2) {
                 if (c > 0) {   // the second pair of a four-feature level
-                    const bool even = grid_even && d[2] % 2 == 0 && d[5] % 2 == 0;
+                    const bool even = grid_even && ((d[2] | d[5]) & 1) == 0;
 #pragma unroll
                     for (int k = 0; k < 4; ++k) g[q][k] = row_pair(a, d, row[q][k], c, true, even);
                 }
